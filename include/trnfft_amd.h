@@ -236,6 +236,18 @@ int tfa_complex_gemm_batched(int64_t batch, int64_t m, int64_t n, int64_t k, con
                              const float* bias_im, float* c_re, float* c_im, int64_t ldc, int64_t stride_c,
                              tfa_stream stream);
 
+/*
+ * tfa_complex_gemm_batched with scratch memory: a product of few output tiles and a long k (a
+ * weight gradient) is summed over several k ranges at once, whose partial results `workspace`
+ * (device memory of tfa_complex_gemm_workspace_size bytes, 0 for every other product; NULL: no
+ * split) holds until a second launch adds them in a fixed order.
+ */
+int tfa_complex_gemm_workspace_size(int64_t batch, int64_t m, int64_t n, int64_t k, size_t* bytes);
+int tfa_complex_gemm_ws(int64_t batch, int64_t m, int64_t n, int64_t k, const float* a_re, const float* a_im,
+                        int64_t lda, int64_t stride_a, int32_t a_op, const float* b_re, const float* b_im, int64_t ldb,
+                        int64_t stride_b, int32_t b_op, float alpha, const float* bias_re, const float* bias_im,
+                        float* c_re, float* c_im, int64_t ldc, int64_t stride_c, void* workspace, tfa_stream stream);
+
 /* Thread-local message describing the last failure on this thread ("" if none). */
 const char* tfa_last_error(void);
 

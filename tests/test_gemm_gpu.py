@@ -155,3 +155,54 @@ def test_dft_gemm_threshold_routing():
         fc._DFT_GEMM_THRESHOLD = old
     ref = oracle.fft_core(re, im, False)
     assert rel_l2(got.real, got.imag, *ref) <= tol_pow2(256)
+
+
+@pytest.mark.parametrize("batch,m,k,n", [
+    (1, 33, 256, 35),      # the shortest split: two ranges of 128, one partial tile
+    (1, 129, 1030, 130),   # four tiles, ragged last range, odd columns (scalar reduction)
+    (1, 1024, 8192, 1024),  # a weight gradient: eight ranges
+    (3, 40, 515, 64),      # batched, last range of three columns
+])
+@pytest.mark.parametrize("a_op,b_op", [(0, 0), (0, 1), (1, 3), (2, 0)])
+def test_gemm_split_k_vs_float64(batch, m, k, n, a_op, b_op):
+    # products of few output tiles are summed in several k ranges (workspace) and reduced
+    import ctypes
+
+    from trnfft_amd import _lib
+    from trnfft_amd.dispatch import gemm_batched
+
+    nbytes = ctypes.c_size_t()
+    assert _lib.lib().tfa_complex_gemm_workspace_size(batch, m, n, k, ctypes.byref(nbytes)) == _lib.TFA_OK
+    assert nbytes.value >= 2 * 8 * batch * m * n
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+
+    def stored(rows, cols, op):
+        shape = (batch, cols, rows) if op in (1, 2) else (batch, rows, cols)
+        return tuple(torch.randn(*shape, generator=g, device="cuda") for _ in range(2))
+
+    def applied(p, op):
+        z = torch.complex(p[0].double(), p[1].double())
+        z = z.transpose(1, 2) if op in (1, 2) else z
+        return (z.conj() if op in (2, 3) else z).resolve_conj().contiguous()
+
+    a, b = stored(m, k, a_op), stored(k, n, b_op)
+    c_re, c_im = gemm_batched(*a, a_op, *b, b_op, batch, alpha=0.5)
+    ref = 0.5 * torch.stack([x @ y for x, y in zip(applied(a, a_op), applied(b, b_op))])
+    assert rel_l2(c_re, c_im, ref.real, ref.imag) <= _tol_k(k), (m, k, n)
+
+
+def test_gemm_split_k_bias_matches_unsplit():
+    from trnfft_amd import _lib
+    from trnfft_amd.dispatch import gemm_ex, ptr, stream_handle
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a, b = (tuple(torch.randn(*s, generator=g, device="cuda") for _ in range(2)) for s in ((70, 700), (50, 700)))
+    bias = tuple(torch.randn(50, generator=g, device="cuda") for _ in range(2))
+    got = gemm_ex(*a, _lib.OP_N, *b, _lib.OP_T, 1.0, *bias)
+    ref = tuple(torch.empty(70, 50, device="cuda") for _ in range(2))
+    rc = _lib.lib().tfa_complex_gemm_ex(70, 50, 700, ptr(a[0]), ptr(a[1]), 700, _lib.OP_N, ptr(b[0]), ptr(b[1]), 700,
+                                        _lib.OP_T, 1.0, ptr(bias[0]), ptr(bias[1]), ptr(ref[0]), ptr(ref[1]), 50,
+                                        stream_handle(a[0].device))
+    _lib.check(rc, "tfa_complex_gemm_ex")
+    # two fp32 sums of the same 1400 products in another order
+    assert rel_l2(*got, *ref) <= 2 * _tol_k(700)

@@ -353,7 +353,9 @@ struct GemmArgs {
   hipStream_t stream;
   long long batch = 1;            // matrix triples (grid.y)
   long long sa = 0, sb = 0, sc = 0;  // batch strides in floats (0: operand shared by the batch)
+  float* workspace = nullptr;        // cgemm_workspace_bytes of scratch, or nullptr: K is not split
 };
 hipError_t launch_cgemm(const GemmArgs& a);
+size_t cgemm_workspace_bytes(long long batch, long long m, long long n, long long k);
 
 }  // namespace tfa

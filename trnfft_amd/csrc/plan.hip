@@ -1102,6 +1102,22 @@ int tfa_complex_gemm_batched(int64_t batch, int64_t m, int64_t n, int64_t k, con
                              int64_t ldb, int64_t stride_b, int32_t b_op, float alpha, const float* bias_re,
                              const float* bias_im, float* c_re, float* c_im, int64_t ldc, int64_t stride_c,
                              tfa_stream stream) {
+  return tfa_complex_gemm_ws(batch, m, n, k, a_re, a_im, lda, stride_a, a_op, b_re, b_im, ldb, stride_b, b_op, alpha,
+                             bias_re, bias_im, c_re, c_im, ldc, stride_c, nullptr, stream);
+}
+
+int tfa_complex_gemm_workspace_size(int64_t batch, int64_t m, int64_t n, int64_t k, size_t* bytes) {
+  if (!bytes) return fail(TFA_ERR_INVALID, "null bytes pointer");
+  if (batch < 0 || m < 0 || n < 0 || k < 0) return fail(TFA_ERR_INVALID, "negative dimension");
+  if (m > INT32_MAX || n > INT32_MAX || k > INT32_MAX) return fail(TFA_ERR_UNSUPPORTED, "dimension above 2^31");
+  *bytes = tfa::cgemm_workspace_bytes(batch, m, n, k);
+  return TFA_OK;
+}
+
+int tfa_complex_gemm_ws(int64_t batch, int64_t m, int64_t n, int64_t k, const float* a_re, const float* a_im,
+                        int64_t lda, int64_t stride_a, int32_t a_op, const float* b_re, const float* b_im, int64_t ldb,
+                        int64_t stride_b, int32_t b_op, float alpha, const float* bias_re, const float* bias_im,
+                        float* c_re, float* c_im, int64_t ldc, int64_t stride_c, void* workspace, tfa_stream stream) {
   if (batch < 0 || m < 0 || n < 0 || k < 0) return fail(TFA_ERR_INVALID, "negative dimension");
   if (stride_a < 0 || stride_b < 0 || stride_c < 0) return fail(TFA_ERR_INVALID, "negative batch stride");
   if (a_op < TFA_OP_N || a_op > TFA_OP_R || b_op < TFA_OP_N || b_op > TFA_OP_R)
@@ -1120,6 +1136,7 @@ int tfa_complex_gemm_batched(int64_t batch, int64_t m, int64_t n, int64_t k, con
   g.sa = stride_a;
   g.sb = stride_b;
   g.sc = stride_c;
+  g.workspace = static_cast<float*>(workspace);
   hipError_t e = tfa::launch_cgemm(g);
   return e == hipSuccess ? TFA_OK : hip_fail(e, "batched complex gemm launch");
 }

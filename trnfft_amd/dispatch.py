@@ -141,6 +141,13 @@ def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
 
 
+def _gemm_workspace(batch: int, m: int, n: int, k: int, dev: torch.device, what: str) -> torch.Tensor | None:
+    """Scratch for a product whose k is summed in several ranges at once (None: not split)."""
+    nbytes = ctypes.c_size_t()
+    _lib.check(_lib.lib().tfa_complex_gemm_workspace_size(batch, m, n, k, ctypes.byref(nbytes)), what)
+    return torch.empty(nbytes.value // 4, dtype=torch.float32, device=dev) if nbytes.value else None
+
+
 def gemm_ex(a_re, a_im, a_op: int, b_re, b_im, b_op: int, alpha: float = 1.0, bias_re=None, bias_im=None,
             what: str = "complex_gemm"):
     """C = alpha * op(A) @ op(B) (+ bias) on the MFMA kernel for 2-D device fp32 planes; returns
@@ -155,10 +162,11 @@ def gemm_ex(a_re, a_im, a_op: int, b_re, b_im, b_op: int, alpha: float = 1.0, bi
         raise ValueError(f"{what}: inner dimensions differ ({k} vs {kb})")
     c_re = torch.empty(m, n, device=dev, dtype=torch.float32)
     c_im = torch.empty(m, n, device=dev, dtype=torch.float32)
+    ws = _gemm_workspace(1, m, n, k, dev, what)
     with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_complex_gemm_ex(
-            m, n, k, ptr(a_re), ptr(a_im), a_re.shape[1], a_op, ptr(b_re), ptr(b_im), b_re.shape[1], b_op,
-            float(alpha), ptr(bias_re), ptr(bias_im), ptr(c_re), ptr(c_im), n, stream_handle(dev),
+        rc = _lib.lib().tfa_complex_gemm_ws(
+            1, m, n, k, ptr(a_re), ptr(a_im), a_re.shape[1], 0, a_op, ptr(b_re), ptr(b_im), b_re.shape[1], 0, b_op,
+            float(alpha), ptr(bias_re), ptr(bias_im), ptr(c_re), ptr(c_im), n, 0, ptr(ws), stream_handle(dev),
         )
     _lib.check(rc, what)
     return c_re, c_im
@@ -181,10 +189,11 @@ def gemm_batched(a_re, a_im, a_op: int, b_re, b_im, b_op: int, batch: int, alpha
     sb = 0 if b_re.shape[0] == 1 else b_re.shape[1] * b_re.shape[2]
     c_re = torch.empty(batch, m, n, device=dev, dtype=torch.float32)
     c_im = torch.empty(batch, m, n, device=dev, dtype=torch.float32)
+    ws = _gemm_workspace(batch, m, n, k, dev, what)
     with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_complex_gemm_batched(
+        rc = _lib.lib().tfa_complex_gemm_ws(
             batch, m, n, k, ptr(a_re), ptr(a_im), a_re.shape[2], sa, a_op, ptr(b_re), ptr(b_im), b_re.shape[2], sb,
-            b_op, float(alpha), ptr(None), ptr(None), ptr(c_re), ptr(c_im), n, m * n, stream_handle(dev),
+            b_op, float(alpha), ptr(None), ptr(None), ptr(c_re), ptr(c_im), n, m * n, ptr(ws), stream_handle(dev),
         )
     _lib.check(rc, what)
     return c_re, c_im
