@@ -158,9 +158,9 @@ def test_dft_gemm_threshold_routing():
 
 
 @pytest.mark.parametrize("batch,m,k,n", [
-    (1, 33, 256, 35),      # the shortest split: two ranges of 128, one partial tile
+    (1, 33, 256, 35),      # one partial tile
     (1, 129, 1030, 130),   # four tiles, ragged last range, odd columns (scalar reduction)
-    (1, 1024, 8192, 1024),  # a weight gradient: eight ranges
+    (1, 1024, 8192, 1024),  # a weight gradient
     (3, 40, 515, 64),      # batched, last range of three columns
 ])
 @pytest.mark.parametrize("a_op,b_op", [(0, 0), (0, 1), (1, 3), (2, 0)])
@@ -206,3 +206,69 @@ def test_gemm_split_k_bias_matches_unsplit():
     _lib.check(rc, "tfa_complex_gemm_ex")
     # two fp32 sums of the same 1400 products in another order
     assert rel_l2(*got, *ref) <= 2 * _tol_k(700)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 1, 1), (5, 7, 3), (128, 16, 128), (129, 17, 127), (300, 15, 257), (256, 63, 131),
+                                   (700, 130, 900)])
+@pytest.mark.parametrize("a_op,b_op", [(a, b) for a in range(4) for b in range(4)])
+def test_gemm_tile_edges_every_op(m, k, n, a_op, b_op):
+    # tile and stage remainders in every operand order, conjugations included
+    from trnfft_amd.dispatch import gemm_ex
+
+    g = torch.Generator(device="cuda").manual_seed(m * 31 + k)
+
+    def stored(rows, cols, op):
+        shape = (cols, rows) if op in (1, 2) else (rows, cols)
+        return tuple(torch.randn(*shape, generator=g, device="cuda") for _ in range(2))
+
+    def applied(p, op):
+        z = torch.complex(p[0].double().cpu(), p[1].double().cpu())
+        z = z.T if op in (1, 2) else z
+        return z.conj().resolve_conj() if op in (2, 3) else z
+
+    a, b = stored(m, k, a_op), stored(k, n, b_op)
+    got = gemm_ex(*a, a_op, *b, b_op, 0.5)
+    ref = 0.5 * (applied(a, a_op) @ applied(b, b_op))
+    assert rel_l2(*got, ref.real, ref.imag) <= _tol_k(k), (m, k, n)
+
+
+def test_gemm_operands_of_one_sign():
+    # the running sums grow all the way, so a truncating accumulation would show: K / 16 rounded
+    # additions and two truncations per stage of 16, each 2^-24 of the sum at most
+    k = 1024
+    g = torch.Generator(device="cuda").manual_seed(2)
+    a = tuple(torch.rand(512, k, generator=g, device="cuda") for _ in range(2))
+    b = tuple(torch.rand(k, 4096, generator=g, device="cuda") for _ in range(2))
+    got = trnfft_amd.complex_matmul(ComplexTensor(*a), ComplexTensor(*b))
+    ref = oracle.complex_matmul(tuple(t.double() for t in a), tuple(t.double() for t in b))
+    assert rel_l2(got.real, got.imag, *ref) <= 2.0**-24 * (2 + math.sqrt(k / 16))
+
+
+@pytest.mark.parametrize("scale", [2.0**-90, 2.0**-110, 2.0**-122, 2.0**100])
+def test_gemm_extreme_magnitudes(scale):
+    # operands whose bf16 pieces would be denormal keep fp32 precision
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = tuple(torch.randn(200, 70, generator=g, device="cuda") * scale for _ in range(2))
+    b = tuple(torch.randn(70, 150, generator=g, device="cuda") for _ in range(2))
+    got = trnfft_amd.complex_matmul(ComplexTensor(*a), ComplexTensor(*b))
+    ref = oracle.complex_matmul(tuple(t.double() for t in a), tuple(t.double() for t in b))
+    assert rel_l2(got.real.double() / scale, got.imag.double() / scale, ref[0] / scale, ref[1] / scale) <= _tol_k(70)
+
+
+@pytest.mark.parametrize("k", [40, 512])  # without and with a split of k
+def test_gemm_nonfinite_operands(k):
+    # infinities and NaN reach exactly the outputs they reach in fp32 arithmetic
+    g = torch.Generator(device="cuda").manual_seed(4)
+    a = tuple(torch.randn(150, k, generator=g, device="cuda") for _ in range(2))
+    b = tuple(torch.randn(k, 140, generator=g, device="cuda") for _ in range(2))
+    a[0][3, 5] = float("inf")
+    a[1][7, k - 1] = float("nan")
+    b[1][11, 139] = -float("inf")
+    got = trnfft_amd.complex_matmul(ComplexTensor(*a), ComplexTensor(*b))
+    ref = oracle.complex_matmul(tuple(t.double() for t in a), tuple(t.double() for t in b))
+    for x, y in zip((got.real, got.imag), ref):
+        assert torch.equal(torch.isnan(x), torch.isnan(y))
+        assert torch.equal(torch.isposinf(x), torch.isposinf(y))
+        assert torch.equal(torch.isneginf(x), torch.isneginf(y))
+    ok = [torch.isfinite(y) for y in ref]
+    assert rel_l2(got.real[ok[0]], got.imag[ok[1]], ref[0][ok[0]], ref[1][ok[1]]) <= _tol_k(k)

@@ -1,131 +1,369 @@
-// Complex GEMM on the fp32 matrix cores (v_mfma_f32_32x32x2f32), split re/im planes.
+// Complex GEMM on the bf16 matrix cores at fp32 precision (v_mfma_f32_32x32x16_bf16), split re/im planes.
 //
 //   C = alpha * (op(A) @ op(B)) + bias,  op(X) = X, X^T, conj(X)^T or conj(X)
 //   C_re = A_re B_re - A_im B_im,  C_im = A_re B_im + A_im B_re   (on the op'ed operands)
-// A transposed operand is staged through LDS in the same [k][i] layout as a plain one (only the
-// global load pattern differs); conjugation negates the imaginary plane as it is staged.
 //
-// One kernel computes all four real products: each k-step loads the A_re/A_im and B_re/B_im
-// fragments once from LDS and issues four MFMAs into two accumulator sets (the NKI kernel's
-// "stationary reuse" idea, trnfft/nki/dispatch.py:121-200 and :267-345, in CDNA4 form).
-// Workgroup tile 128 x 128 (per plane), 4 waves of 64 x 64, BK = 16 k per LDS stage with the
-// next stage prefetched into registers while the current one is consumed.
+// Every fp32 operand is the exact sum of three bf16 pieces of 8 significant bits each (x1 = the top
+// 16 bits of x, x2 = those of x - x1, x3 = x - x1 - x2), so a product a b is the sum of nine bf16
+// products, each exact in fp32; the six of a weight of 2^-16 or more (a1 b1, a1 b2, a2 b1, a2 b2, a1 b3,
+// a3 b1) run on the matrix cores into fp32 accumulators, the other three are below 2^-24 of a b.
+// Against 64 bits (random normal operands, relative 2-norm) that is closer than fp32 products were: 1.7e-7
+// against 8.1e-7 at K = 1024, 8e-8 against 1.45e-7 at K = 33.  The matrix rate is what pays for it: 8192 x
+// 1024 x 1024 takes 325 us back to back (515 with v_mfma_f32_32x32x2f32 at 85 % of its peak), 412 GF of bf16
+// products at 1.27 PF; the matrix cores are busy 68 % of the cycles, at the 1.66 GHz that the card then
+// runs at (rocprofv3; the same work spread thinner clocked higher: 52 % busy, 1.95 GHz, 10 % slower).
+//
+// One kernel computes all four real products: each k-step loads the fragments of the three pieces of
+// A_re/A_im and B_re/B_im once from LDS for 24 MFMAs per 32 x 32 tile of the two accumulator sets (the
+// NKI kernel's "stationary reuse" idea, trnfft/nki/dispatch.py:121-200 and :267-345, in CDNA4 form).
+// Workgroup tile 128 x 128 (per plane), 8 waves of 64 x 32, 16 k per stage, two stages in LDS (one
+// barrier per stage): while one stage is multiplied the next is split and stored, and the one after
+// it is on its way from memory in registers.  Waves w and w + 4 share a SIMD; one of them splits before
+// its MFMAs and the other after, so that the matrix core has work throughout.
 #include <algorithm>
+#include <utility>
 
 #include "kernels.h"
 
 namespace tfa {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int GBM = 128, GBN = 128, GBK = 16;
-constexpr int GLD = GBM + 2;  // LDS row pitch in floats (pad 2: transposed stores hit distinct banks)
+constexpr int kThreads = 512;
+typedef floatx16 Acc[2];  // a wave's 64 x 32 sums of one plane
 
-// Global -> register tile loads. A tile: GBM rows x GBK k (k contiguous in memory). Thread t
-// covers row t/2, k offset (t%2)*8: 8 floats per plane.
-struct ATile {
-  float re[8], im[8];
+// A stage of one operand is 128 rows x 16 k x 2 planes: a thread holds eight k (half) of one row of one plane.
+//   k contiguous in memory (plain A, transposed B): lanes 2r and 2r + 1 hold the halves of row r,
+//   so a row's 64 bytes are one run;
+//   rows contiguous (transposed A, plain B): lanes run over the rows, a wave's load instruction
+//   covers 64 consecutive floats of one k.
+template <bool KMAJOR>
+struct Slot {
+  int plane, row, half;
+  __device__ __forceinline__ Slot(int t, int w) {  // w: the wave (uniform)
+    plane = w >> 2;
+    row = KMAJOR ? (t & 255) >> 1 : t & 127;
+    half = KMAJOR ? t & 1 : (w >> 1) & 1;
+  }
 };
 
-__device__ __forceinline__ void load_kmajor_tile(const float* __restrict__ P_re, const float* __restrict__ P_im,
-                                                 long long ld, int rows, int K, int row0, int k0, int t,
-                                                 bool vec_ok, ATile& o) {
-  const int r = row0 + t / 2;
-  const int kq = k0 + (t % 2) * 8;
-  if (r < rows && vec_ok && kq + 8 <= K) {
-    const float4* pr = reinterpret_cast<const float4*>(P_re + (size_t)r * ld + kq);
-    const float4* pi = reinterpret_cast<const float4*>(P_im + (size_t)r * ld + kq);
-    float4 a = pr[0], b = pr[1], c = pi[0], d = pi[1];
-    o.re[0] = a.x; o.re[1] = a.y; o.re[2] = a.z; o.re[3] = a.w;
-    o.re[4] = b.x; o.re[5] = b.y; o.re[6] = b.z; o.re[7] = b.w;
-    o.im[0] = c.x; o.im[1] = c.y; o.im[2] = c.z; o.im[3] = c.w;
-    o.im[4] = d.x; o.im[5] = d.y; o.im[6] = d.z; o.im[7] = d.w;
-  } else {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const bool in = r < rows && kq + c < K;
-      o.re[c] = in ? P_re[(size_t)r * ld + kq + c] : 0.0f;
-      o.im[c] = in ? P_im[(size_t)r * ld + kq + c] : 0.0f;
-    }
-  }
-}
+// four consecutive floats at any float's alignment
+struct __attribute__((packed, aligned(4))) Quad {
+  float x, y, z, w;
+};
 
-// B tile for the non-transposed case: GBK k-rows x GBN columns (n contiguous). Thread t covers
-// k row t/16, columns (t%16)*8 .. +8.
-__device__ __forceinline__ void load_nmajor_tile(const float* __restrict__ P_re, const float* __restrict__ P_im,
-                                                 long long ld, int N, int K, int col0, int k0, int t,
-                                                 bool vec_ok, ATile& o) {
-  const int k = k0 + t / 16;
-  const int j = col0 + (t % 16) * 8;
-  if (k < K && vec_ok && j + 8 <= N) {
-    const float4* pr = reinterpret_cast<const float4*>(P_re + (size_t)k * ld + j);
-    const float4* pi = reinterpret_cast<const float4*>(P_im + (size_t)k * ld + j);
-    float4 a = pr[0], b = pr[1], c = pi[0], d = pi[1];
-    o.re[0] = a.x; o.re[1] = a.y; o.re[2] = a.z; o.re[3] = a.w;
-    o.re[4] = b.x; o.re[5] = b.y; o.re[6] = b.z; o.re[7] = b.w;
-    o.im[0] = c.x; o.im[1] = c.y; o.im[2] = c.z; o.im[3] = c.w;
-    o.im[4] = d.x; o.im[5] = d.y; o.im[6] = d.z; o.im[7] = d.w;
-  } else {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const bool in = k < K && j + c < N;
-      o.re[c] = in ? P_re[(size_t)k * ld + j + c] : 0.0f;
-      o.im[c] = in ? P_im[(size_t)k * ld + j + c] : 0.0f;
-    }
-  }
-}
-
-// LDS layout: S[plane][k][i] (i contiguous) so an MFMA operand fragment is 32 consecutive floats.
-// `sim` (+1 or -1) multiplies the imaginary plane (conjugation).
-__device__ __forceinline__ void store_kmajor(float (*S)[GBK][GLD], int t, const ATile& o, float sim) {
-  const int r = t / 2, kq = (t % 2) * 8;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    S[0][kq + c][r] = o.re[c];
-    S[1][kq + c][r] = o.im[c] * sim;
-  }
-}
-
-__device__ __forceinline__ void store_nmajor(float (*S)[GBK][GLD], int t, const ATile& o, float sim) {
-  const int k = t / 16, j = (t % 16) * 8;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    S[0][k][j + c] = o.re[c];
-    S[1][k][j + c] = o.im[c] * sim;
-  }
-}
-
-// Operand staging: A_T = op(A) is a transpose (A stored k x m); B_T = op(B) is a transpose
-// (B stored n x k).  A plain A and a transposed B are k-contiguous; the other two m/n-contiguous.
-template <bool A_T>
-__device__ __forceinline__ void load_a(const float* A_re, const float* A_im, long long lda, int M, int K, int row0,
-                                       int k0, int t, bool vec, ATile& o) {
-  if constexpr (A_T) load_nmajor_tile(A_re, A_im, lda, M, K, row0, k0, t, vec, o);
-  else load_kmajor_tile(A_re, A_im, lda, M, K, row0, k0, t, vec, o);
-}
-template <bool B_T>
-__device__ __forceinline__ void load_b(const float* B_re, const float* B_im, long long ldb, int N, int K, int col0,
-                                       int k0, int t, bool vec, ATile& o) {
-  if constexpr (B_T) load_kmajor_tile(B_re, B_im, ldb, N, K, col0, k0, t, vec, o);
-  else load_nmajor_tile(B_re, B_im, ldb, N, K, col0, k0, t, vec, o);
-}
+// One operand's tile: 128 rows from row0, k below K.  Rows past the last one repeat it: what they add
+// to is not stored.
 template <bool KMAJOR>
-__device__ __forceinline__ void stage(float (*S)[GBK][GLD], int t, const ATile& o, float sim) {
-  if constexpr (KMAJOR) store_kmajor(S, t, o, sim);
-  else store_nmajor(S, t, o, sim);
+struct Operand {
+  const float* P;  // this thread's plane, at its row (k contiguous) or the tile's first row
+  long long ld;
+  int K, col;  // rows contiguous: this thread's row in the tile
+  Slot<KMAJOR> q;
+
+  __device__ __forceinline__ Operand(const float* re, const float* im, long long ld_, int rows, int K_, int row0,
+                                     int t, int w)
+      : ld(ld_), K(K_), q(t, w) {
+    const int left = rows - 1 - row0;
+    col = q.row < left ? q.row : left;
+    P = (q.plane ? im : re) + (KMAJOR ? (size_t)(row0 + col) * ld : (size_t)row0);
+  }
+  // a whole stage: k0 + GBK <= K
+  __device__ __forceinline__ void load(int k0, float (&x)[8]) const {
+    const int kq = k0 + q.half * 8;
+    if constexpr (KMAJOR) {
+      const Quad* p = reinterpret_cast<const Quad*>(P + kq);
+      const Quad a = p[0], b = p[1];
+      x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+      x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+    } else {
+      const float* p = P + (size_t)kq * ld;
+#pragma unroll
+      for (int c = 0; c < 8; ++c) x[c] = (p + c * ld)[col];
+    }
+  }
+  // the last, partial stage: k at or past K reads as zero
+  __device__ __forceinline__ void load_tail(int k0, float (&x)[8]) const {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const int k = k0 + q.half * 8 + c, kc = k < K ? k : K - 1;
+      x[c] = KMAJOR ? P[kc] : P[(size_t)kc * ld + col];
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (k0 + q.half * 8 + c >= K) x[c] = 0.0f;
+  }
+};
+
+// LDS of the pieces: per operand and plane three blocks, each two halves of the stage's 16 k, a half
+// 128 rows of 8 k (16 bytes).  An MFMA fragment (lane l: row l % 32, half l / 32) is then one ds_read_b128
+// over two contiguous runs; the 64 bytes between the halves keep the k-contiguous stores (lanes alternate
+// between the halves) off each other's banks.
+constexpr int kHalf = GBM * 16 + 64;  // bytes
+constexpr int kPiece = 2 * kHalf;
+constexpr int kPlane = 3 * kPiece;
+constexpr int kOperand = 2 * kPlane;
+constexpr int kStage = 2 * kOperand;
+static_assert(GBM == GBN, "both operands are staged alike");
+
+// Magnitudes below this leave pieces (2^-24 of the value) in the denormal range, which the bf16
+// matrix instructions flush: operands of 1e-36 lost 5e-5 of the result.
+constexpr float kTiny = 0x1p-100f;
+
+// Eight k of one row, split into their three pieces in four steps of two k.
+struct Split {
+  unsigned p[3][4];
+  template <int C>
+  __device__ __forceinline__ void step(const float (&x)[8]) {
+    float r[2] = {x[2 * C], x[2 * C + 1]};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      // the two top halves in one register
+      p[q][C] = __builtin_amdgcn_perm(__float_as_uint(r[1]), __float_as_uint(r[0]), 0x07060302u);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) r[h] -= __uint_as_float(__float_as_uint(r[h]) & 0xffff0000u);
+    }
+  }
+  __device__ __forceinline__ void store(char* dst) const {
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      *reinterpret_cast<uint4*>(dst + q * kPiece) = make_uint4(p[q][0], p[q][1], p[q][2], p[q][3]);
+  }
+};
+
+// Whether all of eight values are below kTiny and not all are zero (a run of such values in a row whose
+// other values are larger costs nothing, as the flushed parts are below 2^-24 of those).
+__device__ __forceinline__ int tiny_run(const float (&x)[8]) {
+  float m = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) m = fmaxf(m, fabsf(x[c]));
+  return m < kTiny && m > 0.0f ? 1 : 0;
 }
 
-template <bool A_T, bool B_T>
-__global__ __launch_bounds__(256, 2) void cgemm_kernel(int M, int N, int K, const float* __restrict__ A_re,
-                                                    const float* __restrict__ A_im, long long lda, float a_sim,
-                                                    const float* __restrict__ B_re, const float* __restrict__ B_im,
-                                                    long long ldb, float b_sim, const float* __restrict__ bias_re,
-                                                    const float* __restrict__ bias_im, float* __restrict__ C_re,
-                                                    float* __restrict__ C_im, long long ldc, float alpha,
-                                                    long long sa, long long sb, long long sc, int k_chunk,
-                                                    long long sz) {
-  __shared__ float As[2][GBK][GLD];
-  __shared__ float Bs[2][GBK][GLD];
+// a sum outside the range in which the pieces' products are those of fp32 (zero is inside)
+__device__ __forceinline__ int outside(float x) {
+  const float m = fabsf(x);
+  return (!(m < INFINITY) ? 1 : 0) | (m < kTiny && m > 0.0f ? 1 : 0);
+}
+
+// a b + c d over one stage's 16 k, from zero and smallest products first: the instruction truncates its
+// sum, and only the last two products meet a sum of full size here.  (Chained through the whole of K
+// instead, the truncations add up: operands of one sign 2.4e-6 from 64 bits at K = 1024, against
+// 6.0e-7 for fp32 products and 1.1e-7 for these sums added in fp32.)
+// Step S of 12 is one MFMA of each of two chains: im += A_re B_im + A_im B_re, re += A_re B_re - A_im B_im.
+template <int S>
+__device__ __forceinline__ void product_step(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], const bf16x8 (&nb)[3],
+                                             floatx16& im, floatx16& re) {
+  constexpr int P[6] = {2, 0, 1, 1, 0, 0}, Q[6] = {0, 2, 1, 0, 1, 0};
+  constexpr int p = S < 5 ? S : S < 10 ? S - 5 : 5;  // pieces
+  if constexpr (S == 0) im = re = floatx16{};
+  if constexpr (S < 5 || S == 10) {
+    im = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][P[p]], b[1][Q[p]], im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][P[p]], b[0][Q[p]], re, 0, 0, 0);
+  } else {
+    im = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][P[p]], b[0][Q[p]], im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][P[p]], nb[Q[p]], re, 0, 0, 0);
+  }
+}
+
+__device__ __forceinline__ void load_frags(const char* S, bf16x8 (&f)[2][3]) {
+#pragma unroll
+  for (int p = 0; p < 6; ++p)
+    f[p / 3][p % 3] = *reinterpret_cast<const bf16x8*>(S + (p / 3) * kPlane + (p % 3) * kPiece);
+}
+
+__device__ __forceinline__ bf16x8 negated(bf16x8 v) {
+  uint4 u = __builtin_bit_cast(uint4, v);
+  u.x ^= 0x80008000u; u.y ^= 0x80008000u; u.z ^= 0x80008000u; u.w ^= 0x80008000u;
+  return __builtin_bit_cast(bf16x8, u);
+}
+
+template <int... I, class F>
+__device__ __forceinline__ void unroll_impl(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// f(0), ..., f(N - 1) with constant arguments
+template <int N, class F>
+__device__ __forceinline__ void unroll(F&& f) {
+  unroll_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
+__device__ __forceinline__ void clear(Acc& acc) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
+}
+
+// The tile's sums with fp32 products (v_mfma_f32_32x32x2f32), k from k_begin to K: the pieces of an
+// infinity are not its sum and those of the smallest numbers are flushed, so a workgroup that met either
+// (or an overflow) takes this path over, and its results are those of fp32 arithmetic.
+constexpr int GLD = GBM + 2;  // LDS row pitch in floats (pad 2: transposed stores hit distinct banks)
+static_assert(2 * kStage >= 2 * 2 * GBK * GLD * (int)sizeof(float), "staged in the same LDS");
+
+template <bool CONJ_B, class OpA, class OpB>
+__device__ __forceinline__ void tile_f32(float (*As)[GBK][GLD], float (*Bs)[GBK][GLD], int k_begin, const OpA& A,
+                                         const OpB& B, int w, Acc& acc_re, Acc& acc_im) {
+  const int lane = threadIdx.x & 63, wm = w >> 2, wn = w & 3, li = lane & 31, lk = lane >> 5;
+  for (int k0 = k_begin; k0 < A.K; k0 += GBK) {
+    float xa[8], xb[8];
+    if (k0 + GBK <= A.K) {
+      A.load(k0, xa);
+      B.load(k0, xb);
+    } else {
+      A.load_tail(k0, xa);
+      B.load_tail(k0, xb);
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      As[A.q.plane][A.q.half * 8 + c][A.q.row] = xa[c];
+      Bs[B.q.plane][B.q.half * 8 + c][B.q.row] = xb[c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int kk = 0; kk < GBK; kk += 2) {
+      const float br = Bs[0][kk + lk][wn * 32 + li], b1 = Bs[1][kk + lk][wn * 32 + li];
+      const float bi = CONJ_B ? -b1 : b1;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const float ar = As[0][kk + lk][wm * 64 + i * 32 + li], ai = As[1][kk + lk][wm * 64 + i * 32 + li];
+        acc_re[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ar, br, acc_re[i], 0, 0, 0);
+        acc_re[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(-ai, bi, acc_re[i], 0, 0, 0);
+        acc_im[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ar, bi, acc_im[i], 0, 0, 0);
+        acc_im[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ai, br, acc_im[i], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The tile's sums with split products, k from k_begin to K; returns whether this thread met values that
+// need the fp32 path.
+template <bool CONJ_B, class OpA, class OpB>
+__device__ __forceinline__ int tile_split(char* smem, int k_begin, const OpA& A, const OpB& B, int w, Acc& acc_re,
+                                          Acc& acc_im) {
+  const int lane = threadIdx.x & 63, wm = w >> 2, wn = w & 3;
+  const int foff = (lane >> 5) * kHalf + (lane & 31) * 16;
+  const int a_off = foff + wm * 64 * 16, b_off = kOperand + foff + wn * 32 * 16;
+  const int a_dst = A.q.plane * kPlane + A.q.half * kHalf + A.q.row * 16;
+  const int b_dst = kOperand + B.q.plane * kPlane + B.q.half * kHalf + B.q.row * 16;
+  float xa[8], xb[8];
+  int odd = 0;
+  const auto stage = [&](char* S) {
+    Split sa, sb;
+    unroll<4>([&](auto c) {
+      sa.step<c>(xa);
+      sb.step<c>(xb);
+    });
+    odd |= tiny_run(xa) | tiny_run(xb);
+    sa.store(S + a_dst);
+    sb.store(S + b_dst);
+  };
+  // conj(B) swaps B_im and -B_im
+  const auto load_b = [&](const char* S, bf16x8 (&b)[2][3], bf16x8 (&nb)[3]) {
+    load_frags(S + b_off, b);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      nb[q] = negated(b[1][q]);
+      if constexpr (CONJ_B) {
+        const bf16x8 t = b[1][q];
+        b[1][q] = nb[q];
+        nb[q] = t;
+      }
+    }
+  };
+  const int k_whole = k_begin + (A.K - k_begin) / GBK * GBK;  // end of the whole stages
+  int par = 0;
+  if (k_whole > k_begin) {
+    const int k_last = k_whole - GBK;
+    const auto next = [&](int k) { return k < k_last ? k : k_last; };  // (past the end: repeated, unused)
+    A.load(k_begin, xa);
+    B.load(k_begin, xb);
+    stage(smem);
+    A.load(next(k_begin + GBK), xa);
+    B.load(next(k_begin + GBK), xb);
+    __syncthreads();
+    // Each MFMA pair is followed by the VALU work that fits in its shadow (about 12 instructions of 4
+    // cycles in 64), pinned there by the scheduling barriers: the previous stage's sums of the second
+    // row half, then the splitting of the next stage and the sums of the first row half.
+    floatx16 im0, re0, im1 = {}, re1 = {};
+    for (int k0 = k_begin; k0 < k_whole; k0 += GBK, par ^= kStage) {
+      char* const cur = smem + par;
+      char* const nxt = smem + (par ^ kStage);
+      bf16x8 a[2][3], b[2][3], nb[3];
+      load_b(cur, b, nb);
+      load_frags(cur + a_off, a);
+      unroll<12>([&](auto s) {
+        product_step<s>(a, b, nb, im0, re0);
+        if constexpr (s < 8) {
+#pragma unroll
+          for (int r = 2 * s; r < 2 * s + 2; ++r) {
+            acc_im[1][r] += im1[r];
+            acc_re[1][r] += re1[r];
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      load_frags(cur + a_off + 32 * 16, a);
+      Split sa, sb;
+      unroll<12>([&](auto s) {
+        product_step<s>(a, b, nb, im1, re1);
+        if constexpr (s < 4) sa.step<s>(xa);
+        else if constexpr (s < 8) sb.step<s - 4>(xb);
+        if constexpr (s == 4) sa.store(nxt + a_dst);
+        if constexpr (s == 8) {
+          sb.store(nxt + b_dst);
+          odd |= tiny_run(xa) | tiny_run(xb);
+        }
+        if constexpr (s >= 8) {
+#pragma unroll
+          for (int r = 4 * (s - 8); r < 4 * (s - 7); ++r) {
+            acc_im[0][r] += im0[r];
+            acc_re[0][r] += re0[r];
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      A.load(next(k0 + 2 * GBK), xa);
+      B.load(next(k0 + 2 * GBK), xb);
+      __syncthreads();
+    }
+    acc_im[1] += im1;
+    acc_re[1] += re1;
+  }
+  if (k_whole < A.K) {  // the partial stage
+    char* const S = smem + par;
+    A.load_tail(k_whole, xa);
+    B.load_tail(k_whole, xb);
+    stage(S);
+    __syncthreads();
+    bf16x8 a[2][3], b[2][3], nb[3];
+    load_b(S, b, nb);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      floatx16 im, re;
+      load_frags(S + a_off + i * 32 * 16, a);
+      unroll<12>([&](auto s) { product_step<s>(a, b, nb, im, re); });
+      acc_im[i] += im;
+      acc_re[i] += re;
+    }
+  }
+  return odd;
+}
+
+// Operands: A_T = op(A) is a transpose (A stored k x m), B_T = op(B) is one (B stored n x k).  Conjugation:
+// conj(A) op(B) = conj(A conj(op(B))), so CONJ_B is that of exactly one operand, and im_sign is -1 where
+// A is conjugated.
+template <bool A_T, bool B_T, bool CONJ_B>
+__global__ __launch_bounds__(kThreads, 2) void cgemm_kernel(
+    int M, int N, int K, const float* __restrict__ A_re, const float* __restrict__ A_im, long long lda,
+    const float* __restrict__ B_re, const float* __restrict__ B_im, long long ldb, float im_sign,
+    const float* __restrict__ bias_re, const float* __restrict__ bias_im, float* __restrict__ C_re,
+    float* __restrict__ C_im, long long ldc, float alpha, long long sa, long long sb, long long sc, int k_chunk,
+    long long sz) {
+  __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
   // batched products: blockIdx.y selects the matrix triple (batch strides in floats; a stride of 0
   // broadcasts one operand over the batch)
   {
@@ -141,85 +379,46 @@ __global__ __launch_bounds__(256, 2) void cgemm_kernel(int M, int N, int K, cons
   const int k_begin = (int)blockIdx.z * k_chunk;
   K = K - k_begin < k_chunk ? K : k_begin + k_chunk;
   const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int w = t >> 6;
-  const int wm = w >> 1, wn = w & 1;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int wm = w >> 2, wn = w & 3;
   // XCD-aware: neighbouring row tiles (which share B) run on one XCD
   const long long tiles_n = (N + GBN - 1) / GBN;
   const long long tile = xcd_tile_remap(blockIdx.x, gridDim.x);
   const int row0 = (int)(tile / tiles_n) * GBM;
   const int col0 = (int)(tile % tiles_n) * GBN;
-  const bool a_vec = (lda % 4 == 0) && ((reinterpret_cast<size_t>(A_re) | reinterpret_cast<size_t>(A_im)) % 16 == 0);
-  const bool b_vec = (ldb % 4 == 0) && ((reinterpret_cast<size_t>(B_re) | reinterpret_cast<size_t>(B_im)) % 16 == 0);
 
-  floatx16 acc_re[2][2], acc_im[2][2];
+  Acc acc_re, acc_im;
+  clear(acc_re);
+  clear(acc_im);
+  const Operand<!A_T> A(A_re, A_im, lda, M, K, row0, t, w);
+  const Operand<B_T> B(B_re, B_im, ldb, N, K, col0, t, w);
+  int odd = tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im);
+  // non-finite sums, or sums so small that pieces of the products were flushed
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        acc_re[i][j][r] = 0.0f;
-        acc_im[i][j][r] = 0.0f;
-      }
-
-  ATile pa, pb;
-  load_a<A_T>(A_re, A_im, lda, M, K, row0, k_begin, t, a_vec, pa);
-  load_b<B_T>(B_re, B_im, ldb, N, K, col0, k_begin, t, b_vec, pb);
-
-  const int li = lane & 31;
-  const int lk = lane >> 5;
-  for (int k0 = k_begin; k0 < K; k0 += GBK) {
-    stage<!A_T>(As, t, pa, a_sim);
-    stage<B_T>(Bs, t, pb, b_sim);
-    __syncthreads();
-    if (k0 + GBK < K) {
-      load_a<A_T>(A_re, A_im, lda, M, K, row0, k0 + GBK, t, a_vec, pa);
-      load_b<B_T>(B_re, B_im, ldb, N, K, col0, k0 + GBK, t, b_vec, pb);
-    }
-#pragma unroll
-    for (int kk = 0; kk < GBK; kk += 2) {
-      float ar[2], ai[2], nai[2], br[2], bi[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        ar[i] = As[0][kk + lk][wm * 64 + i * 32 + li];
-        ai[i] = As[1][kk + lk][wm * 64 + i * 32 + li];
-        nai[i] = -ai[i];
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        br[j] = Bs[0][kk + lk][wn * 64 + j * 32 + li];
-        bi[j] = Bs[1][kk + lk][wn * 64 + j * 32 + li];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          acc_re[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ar[i], br[j], acc_re[i][j], 0, 0, 0);
-          acc_re[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(nai[i], bi[j], acc_re[i][j], 0, 0, 0);
-          acc_im[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ar[i], bi[j], acc_im[i][j], 0, 0, 0);
-          acc_im[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(ai[i], br[j], acc_im[i][j], 0, 0, 0);
-        }
-    }
-    __syncthreads();
+    for (int r = 0; r < 16; ++r) odd |= outside(acc_re[i][r]) | outside(acc_im[i][r]);
+  if (__syncthreads_or(odd)) {
+    clear(acc_re);
+    clear(acc_im);
+    auto* S = reinterpret_cast<float (*)[GBK][GLD]>(smem);
+    tile_f32<CONJ_B>(S, S + 2, k_begin, A, B, w, acc_re, acc_im);
   }
+  const int li = t & 31, lk = (t >> 5) & 1;
 
-  // D layout of v_mfma_f32_32x32x2f32: lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4, col l%32
+  // D layout of both MFMAs: lane l, register r -> row 8*(r/4) + 4*(l/32) + r%4, col l%32
+  const int col = col0 + wn * 32 + li;
+  if (col >= N) return;
+  const float b_re = bias_re ? bias_re[col] : 0.0f;
+  const float b_im = bias_im ? bias_im[col] : 0.0f;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int col = col0 + wn * 64 + j * 32 + li;
-      if (col >= N) continue;
-      const float b_re = bias_re ? bias_re[col] : 0.0f;
-      const float b_im = bias_im ? bias_im[col] : 0.0f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = row0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-        if (row < M) {
-          C_re[(size_t)row * ldc + col] = acc_re[i][j][r] * alpha + b_re;
-          C_im[(size_t)row * ldc + col] = acc_im[i][j][r] * alpha + b_im;
-        }
+    for (int r = 0; r < 16; ++r) {
+      const int row = row0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
+      if (row < M) {
+        C_re[(size_t)row * ldc + col] = acc_re[i][r] * alpha + b_re;
+        C_im[(size_t)row * ldc + col] = acc_im[i][r] * (alpha * im_sign) + b_im;
       }
     }
 }
@@ -262,24 +461,32 @@ __global__ __launch_bounds__(256) void cgemm_reduce_kernel(const float* __restri
 
 constexpr long long kMaxGridY = 65535;
 
-// Number of K ranges a product is summed in (1: no split).  A workgroup computes one 128 x 128
-// tile, and the chip holds 512 of them (two per CU); a product of fewer than 256 tiles leaves CUs
-// idle, so its K is split until about 512 workgroups run, each over at least kMinSplitK columns.
-// Weight gradients are such products: (1024 x 8192) x (8192 x 1024) is 64 tiles, 2287 us unsplit,
-// 531 us in 8 ranges with their reduction; 220 x 2019 x 334 919 -> 83 us (15 ranges), 1000 x 256 x 1000
-// 84 -> 57 (2 ranges).  The shorter sums also round less (2.3e-6 -> 8.1e-7 at K = 8192).
-constexpr int kMinSplitK = 128;
+// Number of K ranges a product is summed in (1: no split).  A workgroup computes one 128 x 128 tile, one
+// per CU at a time, so the product takes ceil(tiles * ranges / 256) rounds of (K / ranges) / 16 stages of
+// about 2 us; a split adds the launch that reduces the partials (4 us and their traffic at 4 TB/s).  The
+// number with the least sum of these is taken, each range at least kMinSplitK columns.  Weight gradients
+// are such products: (1024 x 8192) x (8192 x 1024) is 64 tiles, 883 us unsplit, 331 us in
+// 4 ranges; 220 x 2019 x 334 227 -> 33 us (26 ranges), 1000 x 256 x 1000 40 -> 30 (4); 1500 x 2048 x 1800, 180
+// tiles, 256 -> 263.
+// The shorter sums also round less (4.4e-7 -> 2.6e-7 at K = 8192).
+constexpr int kMinSplitK = 64;
 int cgemm_splits(long long batch, long long m, long long n, long long k, int* k_chunk) {
   const long long tiles = ((m + GBM - 1) / GBM) * ((n + GBN - 1) / GBN) * batch;
-  long long s = tiles > 0 && tiles < kNumCUs ? 2 * kNumCUs / tiles : 1;
-  s = std::min(s, k / kMinSplitK);
-  if (s < 2 || batch > kMaxGridY) {
-    *k_chunk = (int)k;
-    return 1;
+  *k_chunk = (int)k;
+  if (tiles < 1 || tiles >= kNumCUs || batch > kMaxGridY) return 1;
+  int best = 1;
+  double best_us = (double)((k + GBK - 1) / GBK) * 2.0;
+  for (long long s = 2; s <= k / kMinSplitK && s <= 64; ++s) {
+    const long long chunk = ((k + s - 1) / s + GBK - 1) / GBK * GBK, parts = (k + chunk - 1) / chunk;
+    const double us = (double)((tiles * parts + kNumCUs - 1) / kNumCUs) * (chunk / GBK) * 2.0 + 4.0 +
+                      (double)(parts + 1) * batch * m * n * 8.0 / 4e6;
+    if (us < best_us) {
+      best_us = us;
+      best = (int)parts;
+      *k_chunk = (int)chunk;
+    }
   }
-  const long long c = ((k + s - 1) / s + GBK - 1) / GBK * GBK;
-  *k_chunk = (int)c;
-  return (int)((k + c - 1) / c);
+  return best;
 }
 
 size_t cgemm_workspace_bytes(long long batch, long long m, long long n, long long k) {
@@ -288,18 +495,17 @@ size_t cgemm_workspace_bytes(long long batch, long long m, long long n, long lon
   return s > 1 ? (size_t)s * batch * m * n * 2 * sizeof(float) : 0;
 }
 
-template <bool A_T, bool B_T>
+template <bool A_T, bool B_T, bool CONJ_B>
 static void launch_cgemm_t(const GemmArgs& a, long long tiles) {
-  const float a_sim = (a.a_op == 2 || a.a_op == 3) ? -1.0f : 1.0f;
-  const float b_sim = (a.b_op == 2 || a.b_op == 3) ? -1.0f : 1.0f;
+  const float im_sign = (a.a_op == 2 || a.a_op == 3) ? -1.0f : 1.0f;
   int k_chunk = (int)a.k;
   const int splits = a.workspace ? cgemm_splits(a.batch, a.m, a.n, a.k, &k_chunk) : 1;
   if (splits > 1) {
     const long long per = a.m * a.n, sz = per * a.batch, plane = sz * splits;
     float* ws = a.workspace;
-    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T>), dim3((unsigned)tiles, (unsigned)a.batch, splits), dim3(256), 0,
-                       a.stream, (int)a.m, (int)a.n, (int)a.k, a.a_re, a.a_im, a.lda, a_sim, a.b_re, a.b_im, a.ldb,
-                       b_sim, nullptr, nullptr, ws, ws + plane, a.n, 1.0f, a.sa, a.sb, per, k_chunk, sz);
+    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T, CONJ_B>), dim3((unsigned)tiles, (unsigned)a.batch, splits), dim3(kThreads),
+                       0, a.stream, (int)a.m, (int)a.n, (int)a.k, a.a_re, a.a_im, a.lda, a.b_re, a.b_im, a.ldb,
+                       im_sign, nullptr, nullptr, ws, ws + plane, a.n, 1.0f, a.sa, a.sb, per, k_chunk, sz);
     // four columns per thread where every row of C starts 16-byte aligned
     const bool v4 = a.n % 4 == 0 && a.ldc % 4 == 0 && a.sc % 4 == 0 &&
                     (reinterpret_cast<size_t>(a.c_re) | reinterpret_cast<size_t>(a.c_im) |
@@ -315,9 +521,9 @@ static void launch_cgemm_t(const GemmArgs& a, long long tiles) {
   }
   for (long long b0 = 0; b0 < a.batch; b0 += kMaxGridY) {
     const unsigned nb = (unsigned)std::min(kMaxGridY, a.batch - b0);
-    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T>), dim3((unsigned)tiles, nb), dim3(256), 0, a.stream, (int)a.m,
-                       (int)a.n, (int)a.k, a.a_re + b0 * a.sa, a.a_im + b0 * a.sa, a.lda, a_sim, a.b_re + b0 * a.sb,
-                       a.b_im + b0 * a.sb, a.ldb, b_sim, a.bias_re, a.bias_im, a.c_re + b0 * a.sc,
+    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T, CONJ_B>), dim3((unsigned)tiles, nb), dim3(kThreads), 0, a.stream, (int)a.m,
+                       (int)a.n, (int)a.k, a.a_re + b0 * a.sa, a.a_im + b0 * a.sa, a.lda, a.b_re + b0 * a.sb,
+                       a.b_im + b0 * a.sb, a.ldb, im_sign, a.bias_re, a.bias_im, a.c_re + b0 * a.sc,
                        a.c_im + b0 * a.sc, a.ldc, a.alpha, a.sa, a.sb, a.sc, k_chunk, 0LL);
   }
 }
@@ -325,13 +531,14 @@ static void launch_cgemm_t(const GemmArgs& a, long long tiles) {
 hipError_t launch_cgemm(const GemmArgs& a) {
   const long long tiles = ((a.m + GBM - 1) / GBM) * ((a.n + GBN - 1) / GBN);
   const bool at = a.a_op == 1 || a.a_op == 2, bt = a.b_op == 1 || a.b_op == 2;
-  if (at) {
-    if (bt) launch_cgemm_t<true, true>(a, tiles);
-    else launch_cgemm_t<true, false>(a, tiles);
-  } else {
-    if (bt) launch_cgemm_t<false, true>(a, tiles);
-    else launch_cgemm_t<false, false>(a, tiles);
-  }
+  const bool conj_b = (a.a_op == 2 || a.a_op == 3) != (a.b_op == 2 || a.b_op == 3);
+  using Launch = void (*)(const GemmArgs&, long long);
+  static constexpr Launch table[2][2][2] = {
+      {{launch_cgemm_t<false, false, false>, launch_cgemm_t<false, false, true>},
+       {launch_cgemm_t<false, true, false>, launch_cgemm_t<false, true, true>}},
+      {{launch_cgemm_t<true, false, false>, launch_cgemm_t<true, false, true>},
+       {launch_cgemm_t<true, true, false>, launch_cgemm_t<true, true, true>}}};
+  table[at][bt][conj_b](a, tiles);
   return hipGetLastError();
 }
 
