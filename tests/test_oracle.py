@@ -312,3 +312,19 @@ def test_stage_parallel_equals_fft_core():
     assert oracle.factorize(1 << 20) == (1024, 1024)
     with pytest.raises(ValueError):
         oracle.factorize(4099)
+
+
+def test_direct_transform_lengths_stay_within_the_parity_bound():
+    # the GPU library transforms these lengths directly (csrc/smooth.h); the reference's chain differs
+    # from the exact transform by its fp32 chirp, which has to stay inside the bound there with margin
+    def smooth(n):
+        for p in (2, 3, 5, 7):
+            while n % p == 0:
+                n //= p
+        return n == 1
+
+    g = torch.Generator().manual_seed(1)
+    for n in [n for n in range(36, 641, 4) if smooth(n) and n & (n - 1)]:
+        re, im = torch.randn(8, n, generator=g), torch.randn(8, n, generator=g)
+        exact = torch.fft.fft(torch.complex(re.double(), im.double()))
+        assert rel_l2(*oracle.fft_core(re, im, False), exact.real, exact.imag) <= 0.85 * 1e-5 * math.log2(n), n

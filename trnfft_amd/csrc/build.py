@@ -28,6 +28,9 @@ SOURCES = [
     "kernels_fft2.hip",
     "kernels_real.hip",
     "kernels_istft.hip",
+    "kernels_smooth_stft.hip",
+    "kernels_smooth_istft.hip",
+    "kernels_smooth_c2c.hip",
 ]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

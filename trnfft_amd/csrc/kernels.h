@@ -32,6 +32,19 @@ __device__ __forceinline__ unsigned xcd_tile_remap32(unsigned i, unsigned g) {
 // and written once, so it should not displace other lines in L2 / the Infinity Cache.
 __device__ __forceinline__ float ld_stream(const float* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_stream(float* p, float v) { __builtin_nontemporal_store(v, p); }
+// two / four consecutive floats at any float's alignment
+struct __attribute__((packed, aligned(4))) Pair {
+  float x, y;
+};
+struct __attribute__((packed, aligned(4))) Quad {
+  float x, y, z, w;
+};
+__device__ __forceinline__ float2 ld_pair(const float* p) {
+  const Pair a = *reinterpret_cast<const Pair*>(p);
+  return make_float2(a.x, a.y);
+}
+__device__ __forceinline__ Quad ld_quad(const float* p) { return *reinterpret_cast<const Quad*>(p); }
+__device__ __forceinline__ void st_quad(float* p, Quad v) { *reinterpret_cast<Quad*>(p) = v; }
 __device__ __forceinline__ void st_stream4(float* p, float4 v) {
   typedef float f4v __attribute__((ext_vector_type(4)));
   const f4v w = {v.x, v.y, v.z, v.w};
@@ -218,6 +231,21 @@ struct StridedBlueArgs {
 };
 hipError_t launch_strided_bluestein(int m, const StridedBlueArgs& a);
 
+// Transforms of smooth lengths (smooth.h): contiguous rows (outer of them), or the strided axis of (outer, n, stride)
+struct SmoothArgs {
+  const float* in_re;
+  const float* in_im;  // nullptr: real input
+  float* out_re;       // may equal in_re (in place)
+  float* out_im;
+  const float2* tw;  // smooth_table(n)
+  long long outer, stride;
+  float scale;
+  bool inverse;
+  hipStream_t stream;
+};
+hipError_t launch_smooth_rows(int n, const SmoothArgs& a);
+hipError_t launch_smooth_strided(int n, const SmoothArgs& a);
+
 // Split (transposed-domain four-step) Bluestein, m = m1 * m2 >= 16384.
 struct BlueSplitArgs {
   const float* in_re;
@@ -257,11 +285,14 @@ struct StftArgs {
   const float2* chirp = nullptr;
   const float2* hs = nullptr;
   int m = 0;
+  // smooth n_fft (smooth.h): tw above is the table of the n_fft/2-point transform, this one W_{n_fft}^k, k <= n_fft/2
+  const float2* twn = nullptr;
   // output planes (batch, n_frames, n_bins) instead of (batch, n_bins, n_frames)
   bool frames_major = false;
 };
 hipError_t launch_stft(int n_fft, const StftArgs& a);
 hipError_t launch_stft_blue(int n_fft, const StftArgs& a);  // a.m != 0
+hipError_t launch_stft_smooth(int n_fft, const StftArgs& a);  // a.twn != nullptr
 
 struct RealArgs {
   const float* in_re;  // forward: (batch, n) real rows; inverse: (batch, n/2+1) bins
@@ -310,10 +341,13 @@ struct IstftArgs {
   const float2* chirp = nullptr;
   const float2* hs = nullptr;
   int m = 0;
+  // smooth n_fft (smooth.h): as in StftArgs
+  const float2* twn = nullptr;
 };
 hipError_t launch_istft(int n_fft, const IstftArgs& a);
 int istft_frames_per_tile(int n_fft, bool two_sided = false);
 hipError_t launch_istft_blue(int n_fft, const IstftArgs& a);  // a.m != 0
+hipError_t launch_istft_smooth(int n_fft, const IstftArgs& a);  // a.twn != nullptr
 
 struct Fft2Args {
   const float* in_re;

@@ -49,11 +49,6 @@ struct Slot {
   }
 };
 
-// four consecutive floats at any float's alignment
-struct __attribute__((packed, aligned(4))) Quad {
-  float x, y, z, w;
-};
-
 // One operand's tile: 128 rows from row0, k below K.  Rows past the last one repeat it: what they add
 // to is not stored.
 template <bool KMAJOR>
@@ -74,8 +69,7 @@ struct Operand {
   __device__ __forceinline__ void load(int k0, float (&x)[8]) const {
     const int kq = k0 + q.half * 8;
     if constexpr (KMAJOR) {
-      const Quad* p = reinterpret_cast<const Quad*>(P + kq);
-      const Quad a = p[0], b = p[1];
+      const Quad a = ld_quad(P + kq), b = ld_quad(P + kq + 4);
       x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
       x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
     } else {

@@ -539,6 +539,7 @@ static hipError_t launch_stft_n(const StftArgs& a) {
 }
 
 hipError_t launch_stft(int n_fft, const StftArgs& a) {
+  if (a.twn) return launch_stft_smooth(n_fft, a);
   if (a.m != 0) return launch_stft_blue(n_fft, a);
   switch (n_fft) {
     case 16: return launch_stft_n<16>(a);

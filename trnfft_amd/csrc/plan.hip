@@ -12,6 +12,7 @@
 
 #include "../../include/trnfft_amd.h"
 #include "kernels.h"
+#include "smooth.h"
 
 using tfa::LdsShape;
 
@@ -67,6 +68,15 @@ std::vector<float2> lds_table(int n, int dir, int e = 0) {
   return t;
 }
 
+// Exchange twiddles of the smooth transform of length n (tfa::Smooth): W_n^(k1 j2) at k1 * N2 + j2.
+std::vector<float2> smooth_table(int n) {
+  const int n1 = tfa::smooth_n1(n), n2 = n / n1;
+  std::vector<float2> t((size_t)n);
+  for (int k = 0; k < n1; ++k)
+    for (int j = 0; j < n2; ++j) t[(size_t)k * n2 + j] = unit_root((int64_t)k * j, n, -1);
+  return t;
+}
+
 struct DevBuf {
   void* p = nullptr;
 };
@@ -118,6 +128,9 @@ struct tfa_plan {
   int64_t m = 0;  // padded length (Bluestein: the reference's, trnfft/plan.py:42), else n
   int64_t mf = 0;  // Bluestein: internal length of the fused kernel (m, or a shorter mixed-radix length)
   C2cTables fwd, inv;  // C2C uses the one for its direction; Bluestein uses both (length m)
+  // smooth lengths (smooth.h): tables of the n-point transform (Bluestein plans) or of the n/2-point one and
+  // W_n^k, k <= n/2 (STFT plans); such plans have none of the chain's tables
+  float2 *sm_tw = nullptr, *sm_twn = nullptr;
   bool blue_fused = false;  // Bluestein: fused one-launch kernel available (m <= 16384)
   bool blue_split = false;  // Bluestein: split three-pass path available (m >= 16384)
   int blue_m1 = 0, blue_m2 = 0, blue_lo_bits = 0;
@@ -493,6 +506,10 @@ int tfa_plan_create(tfa_plan** out, const tfa_plan_desc* desc) {
         rc = fail(TFA_ERR_UNSUPPORTED, "Bluestein padded length above 2^24 not supported");
         break;
       }
+      if (tfa::smooth_len(n)) {
+        rc = p->upload(smooth_table((int)n), &p->sm_tw);
+        break;
+      }
       p->mf = blue_fused_length(n, m);
       p->blue_fused = p->mf <= kMaxLdsN;
       p->blue_split = m >= kMinBlueSplitM;
@@ -597,6 +614,13 @@ int tfa_plan_create(tfa_plan** out, const tfa_plan_desc* desc) {
         }
         const int e = desc->inverse ? tfa::istft_blue_epth((int)m) : tfa::stft_blue_epth((int)m);
         p->m = p->mf = m;
+        if (tfa::smooth_len(n)) {
+          std::vector<float2> w((size_t)n / 2 + 1);
+          for (int64_t k = 0; k <= n / 2; ++k) w[(size_t)k] = unit_root(k, n, -1);
+          if ((rc = p->upload(smooth_table((int)n / 2), &p->sm_tw))) break;
+          rc = p->upload(w, &p->sm_twn);
+          break;
+        }
         p->fwd.n = p->inv.n = m;
         p->fwd.dir = -1;
         p->inv.dir = 1;
@@ -725,7 +749,7 @@ int tfa_plan_workspace_size(const tfa_plan* plan, int64_t batch, size_t* bytes) 
       *bytes = c2c_workspace(plan->d.inverse ? plan->inv : plan->fwd, batch);
       break;
     case TFA_KIND_BLUESTEIN:
-      if (blue_use_split(plan, batch)) *bytes = (size_t)2 * sizeof(float) * (size_t)batch * (size_t)plan->m;
+      if (!plan->sm_tw && blue_use_split(plan, batch)) *bytes = (size_t)2 * sizeof(float) * (size_t)batch * (size_t)plan->m;
       break;
     default:
       break;
@@ -752,6 +776,11 @@ int tfa_execute(const tfa_plan* plan, int64_t batch, const float* in_re, const f
       return run_c2c(plan->d.inverse ? plan->inv : plan->fwd, batch, in_re, in_im, out_re, out_im,
                      workspace, scale, s);
     case TFA_KIND_BLUESTEIN: {
+      if (plan->sm_tw) {
+        const hipError_t se = tfa::launch_smooth_rows(
+            (int)n, {in_re, in_im, out_re, out_im, plan->sm_tw, batch, 1, scale, plan->d.inverse != 0, s});
+        return se == hipSuccess ? TFA_OK : hip_fail(se, "smooth-length launch");
+      }
       tfa::BluesteinArgs a{in_re, in_im, out_re, out_im, plan->chirp, plan->hs, plan->fwd.tw,
                            plan->inv.tw, (int)n, (int)plan->mf, batch, scale, s, plan->blue_wrap};
       hipError_t e;
@@ -909,6 +938,12 @@ int tfa_execute_strided(const tfa_plan* plan, int64_t outer, int64_t stride, con
   note_capture(plan, stream);
   if (blue) {
     const float bscale = plan->d.inverse ? (float)(1.0 / (double)plan->d.n) : 1.0f;
+    if (plan->sm_tw) {
+      const hipError_t se = tfa::launch_smooth_strided(
+          (int)plan->d.n, {in_re, in_im, out_re, out_im, plan->sm_tw, outer, stride, bscale, plan->d.inverse != 0,
+                           static_cast<hipStream_t>(stream)});
+      return se == hipSuccess ? TFA_OK : hip_fail(se, "strided smooth-length launch");
+    }
     tfa::StridedBlueArgs ba{in_re, in_im, out_re, out_im, plan->chirp, plan->b_hs_s, plan->b_tw_sf, plan->b_tw_si,
                             outer, stride, (int)plan->d.n, bscale, static_cast<hipStream_t>(stream)};
     hipError_t be = tfa::launch_strided_bluestein((int)plan->m, ba);
@@ -958,7 +993,10 @@ int tfa_stft_execute(const tfa_plan* plan, int64_t batch, int64_t num_samples, c
   tfa::StftArgs a{signal, window, out_re, out_im, plan->fwd.tw, (int)num_samples, (int)hop,
                   (int)pad, (int)frames, n_bins, batch, scale, static_cast<hipStream_t>(stream)};
   a.frames_major = (plan->d.flags & TFA_STFT_FRAMES_MAJOR) != 0;
-  if (!is_pow2(n_fft)) {
+  if (plan->sm_tw) {
+    a.tw = plan->sm_tw;
+    a.twn = plan->sm_twn;
+  } else if (!is_pow2(n_fft)) {
     a.tw_i = plan->inv.tw;
     a.chirp = plan->chirp;
     a.hs = plan->hs;
@@ -1016,7 +1054,11 @@ int tfa_istft_execute(const tfa_plan* plan, int64_t batch, int64_t n_frames, con
   a.frames_major = (plan->d.flags & TFA_STFT_FRAMES_MAJOR) != 0;
   a.two_sided = two_sided;
   hipError_t e;
-  if (!is_pow2(n_fft)) {
+  if (plan->sm_tw) {
+    a.tw = plan->sm_tw;
+    a.twn = plan->sm_twn;
+    e = tfa::launch_istft_smooth((int)n_fft, a);
+  } else if (!is_pow2(n_fft)) {
     a.blue_tw_f = plan->fwd.tw;
     a.blue_tw_i = plan->inv.tw;
     a.chirp = plan->chirp;
@@ -1056,15 +1098,19 @@ int tfa_stft_backward_execute(const tfa_plan* plan, int64_t batch, int64_t n_fra
     return fail(TFA_ERR_UNSUPPORTED, "signal too long");
   note_capture(plan, stream);
   const double norm = (plan->d.flags & TFA_STFT_NORMALIZED) ? 1.0 / std::sqrt((double)n_fft) : 1.0;
-  // power of two: r2c adjoint = interior bins halved (scale 1/2, bins 0 and n/2 doubled in the kernel)
+  // power of two or smooth: r2c adjoint = interior bins halved (scale 1/2, bins 0 and n/2 doubled in the kernel)
   tfa::IstftArgs a{grad_re, grad_im, window, grad_padded, plan->inv.tw, (int)n_frames, (int)hop, (int)halo,
-                   batch, covered, 0, covered, padded_len, (float)(pow2 ? 0.5 * norm : norm),
+                   batch, covered, 0, covered, padded_len, (float)(pow2 || plan->sm_tw ? 0.5 * norm : norm),
                    static_cast<hipStream_t>(stream)};
   a.adjoint = true;
   a.vec4 = vec4_ok(a, grad_padded);
   a.frames_major = (plan->d.flags & TFA_STFT_FRAMES_MAJOR) != 0;
   hipError_t e;
-  if (pow2) {
+  if (plan->sm_tw) {
+    a.tw = plan->sm_tw;
+    a.twn = plan->sm_twn;
+    e = tfa::launch_istft_smooth((int)n_fft, a);
+  } else if (pow2) {
     e = tfa::launch_istft((int)n_fft, a);
   } else {
     a.blue_tw_f = plan->fwd.tw;

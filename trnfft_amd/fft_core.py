@@ -7,6 +7,8 @@ treating every leading dimension as batch, and returns new tensors:
 * power-of-two n: the LDS-resident Stockham kernel (n <= 16384) or the two-pass four-step
   kernel pair (n > 16384), replacing the radix-2 ``_cooley_tukey`` (:53-117) and the NKI
   Stockham/butterfly chain (:548-1238);
+* multiples of 4 from 36 to 640 without a prime factor above 7: the two-pass direct transform
+  (csrc/smooth.h; the exact transform, which the reference's fp32 chirp misses by 1.15e-7 n);
 * any other n: the fused Bluestein kernel, replacing ``_bluestein`` (:1285-1376), with the chirp
   built from the reference's fp32 angle expression so results agree with the reference;
 * ``_fft_via_gemm`` (:221-251): DFT as one complex GEMM on the matrix cores, taken when
