@@ -203,6 +203,13 @@ int tfa_stft_backward_execute(const tfa_plan* plan, int64_t batch, int64_t n_fra
                               const float* grad_im, const float* window, float* grad_padded, int64_t padded_len,
                               tfa_stream stream);
 
+/*
+ * The reflect padding's adjoint, in place on (batch, pad + length + pad) rows: each kept sample receives the
+ * gradient of its mirror images, so that columns [pad, pad + length) are the gradient of the signal
+ * (the backward of trnfft/api.py:310-313's F.pad).
+ */
+int tfa_stft_fold_edges(int64_t batch, int64_t pad, int64_t length, float* grad_padded, tfa_stream stream);
+
 /* Operand ops of tfa_complex_gemm_ex (BLAS-style, plus conjugation without transpose). */
 #define TFA_OP_N 0 /* op(X) = X          */
 #define TFA_OP_T 1 /* op(X) = X^T        */

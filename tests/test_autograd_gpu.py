@@ -542,3 +542,17 @@ def test_reference_named_autograd_entry_points():
     y_re, y_im = ag.complex_linear_autograd(_leaf(ar), _leaf(ai), _leaf(wr), _leaf(wi))
     Y = torch.complex(ar.double(), ai.double()) @ torch.complex(wr.double(), wi.double()).T
     assert rel_l2(y_re, y_im, Y.real, Y.imag) <= TOL
+
+
+@pytest.mark.parametrize("batch,pad,length", [(1, 1, 2), (3, 4, 5), (2, 4, 9), (2, 4, 10), (5, 200, 201), (4, 512, 4000)])
+def test_fold_edges_is_the_reflect_padding_adjoint(batch, pad, length):
+    # pads from one sample to all but one of the signal: both edges then fold into the same samples
+    from trnfft_amd import fft_core
+
+    g = torch.randn(batch, length + 2 * pad, generator=torch.Generator().manual_seed(pad), dtype=torch.float64)
+    x = torch.zeros(batch, length, dtype=torch.float64, requires_grad=True)
+    (torch.nn.functional.pad(x, (pad, pad), mode="reflect") * g).sum().backward()
+    d = g.float().cuda()
+    fft_core.execute_fold_edges(d, pad, length)
+    # at most three fp32 terms per sample
+    torch.testing.assert_close(d[:, pad : pad + length].cpu(), x.grad.float(), rtol=1e-6, atol=1e-6)

@@ -311,11 +311,9 @@ def _unpad_reflect(d_xp: torch.Tensor, pad: int, length: int) -> torch.Tensor:
     """Adjoint of the reflect padding x_pad[i] = x[pad - i] (i < pad), x_pad[pad + j] = x[j],
     x_pad[pad + L + i] = x[L - 2 - i]: the kept span, with the reflected edges folded back in
     place (a view of d_xp's rows; pad = 0 is the plain prefix)."""
-    d_x = d_xp[:, pad : pad + length]
     if pad:
-        d_x[:, 1 : pad + 1] += d_xp[:, :pad].flip(-1)
-        d_x[:, length - 1 - pad : length - 1] += d_xp[:, pad + length :].flip(-1)
-    return d_x
+        _fc.execute_fold_edges(d_xp, pad, length)
+    return d_xp[:, pad : pad + length]
 
 
 def stft(x, win, n_fft, hop, center, normalized, onesided, num_frames, frames_major=False) -> ComplexTensor:

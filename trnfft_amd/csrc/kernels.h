@@ -345,6 +345,8 @@ struct IstftArgs {
   const float2* twn = nullptr;
 };
 hipError_t launch_istft(int n_fft, const IstftArgs& a);
+// in-place adjoint of the reflect padding on rows of length + 2 * pad samples (0 < pad < length)
+hipError_t launch_fold_reflect(float* x, long long batch, int pad, int length, hipStream_t stream);
 int istft_frames_per_tile(int n_fft, bool two_sided = false);
 hipError_t launch_istft_blue(int n_fft, const IstftArgs& a);  // a.m != 0
 hipError_t launch_istft_smooth(int n_fft, const IstftArgs& a);  // a.twn != nullptr

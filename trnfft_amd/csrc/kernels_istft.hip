@@ -412,4 +412,33 @@ hipError_t launch_istft(int n_fft, const IstftArgs& a) {
   }
 }
 
+// The reflect padding's adjoint on rows of pad + length + pad samples, in place: sample o of the signal (at pad + o)
+// also receives its mirror images pad - o (1 <= o <= pad) and pad + 2 (length - 1) - o (o >= length - 1 - pad).
+// One thread per receiving sample; only the edges are touched (32 x 64000 at pad 512: one launch of 2 us against
+// four torch launches of 14 us over the same samples and their host time).
+__global__ __launch_bounds__(256) void fold_reflect_kernel(float* __restrict__ x, int pad, int length,
+                                                           long long pitch) {
+  float* row = x + (size_t)blockIdx.y * pitch;
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= 2 * pad) return;
+  // the left receivers 1..pad, then those of the right that are not among them
+  const int o = i < pad ? i + 1 : length - 2 - (i - pad);
+  if (o < 0 || o >= length || (i >= pad && o >= 1 && o <= pad)) return;
+  float v = row[pad + o];
+  if (o >= 1 && o <= pad) v += row[pad - o];
+  if (o >= length - 1 - pad && o <= length - 2) v += row[pad + 2 * (length - 1) - o];
+  row[pad + o] = v;
+}
+
+hipError_t launch_fold_reflect(float* x, long long batch, int pad, int length, hipStream_t stream) {
+  const long long pitch = (long long)length + 2LL * pad;
+  constexpr long long kMaxGridY = 65535;
+  for (long long b0 = 0; b0 < batch; b0 += kMaxGridY) {
+    const unsigned nb = (unsigned)(batch - b0 < kMaxGridY ? batch - b0 : kMaxGridY);
+    hipLaunchKernelGGL(fold_reflect_kernel, dim3((2 * pad + 255) / 256, nb), dim3(256), 0, stream, x + b0 * pitch, pad,
+                       length, pitch);
+  }
+  return hipGetLastError();
+}
+
 }  // namespace tfa

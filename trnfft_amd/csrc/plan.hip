@@ -1123,6 +1123,16 @@ int tfa_stft_backward_execute(const tfa_plan* plan, int64_t batch, int64_t n_fra
   return e == hipSuccess ? TFA_OK : hip_fail(e, "stft backward launch");
 }
 
+int tfa_stft_fold_edges(int64_t batch, int64_t pad, int64_t length, float* grad_padded, tfa_stream stream) {
+  if (batch < 0 || pad < 0 || length < 1) return fail(TFA_ERR_INVALID, "bad dimension");
+  if (pad >= length) return fail(TFA_ERR_INVALID, "reflect padding needs more samples than pad");
+  if (length > INT32_MAX / 2) return fail(TFA_ERR_UNSUPPORTED, "signal too long");
+  if (batch == 0 || pad == 0) return TFA_OK;
+  if (!grad_padded) return fail(TFA_ERR_INVALID, "null data pointer");
+  hipError_t e = tfa::launch_fold_reflect(grad_padded, batch, (int)pad, (int)length, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? TFA_OK : hip_fail(e, "edge fold launch");
+}
+
 int tfa_complex_gemm_ex(int64_t m, int64_t n, int64_t k, const float* a_re, const float* a_im, int64_t lda,
                         int32_t a_op, const float* b_re, const float* b_im, int64_t ldb, int32_t b_op, float alpha,
                         const float* bias_re, const float* bias_im, float* c_re, float* c_im, int64_t ldc,

@@ -353,6 +353,15 @@ def execute_stft_backward(g_re: torch.Tensor, g_im: torch.Tensor, win: torch.Ten
     return out
 
 
+def execute_fold_edges(d_xp: torch.Tensor, pad: int, length: int) -> None:
+    """Adjoint of the reflect padding, in place on the contiguous (b, pad + length + pad) device rows."""
+    assert d_xp.is_contiguous() and d_xp.shape[-1] == length + 2 * pad
+    dev = d_xp.device
+    with torch.cuda.device(dev):
+        rc = _lib.lib().tfa_stft_fold_edges(d_xp.shape[0], pad, length, ptr(d_xp), stream_handle(dev))
+    _lib.check(rc, "tfa_stft_fold_edges")
+
+
 def strided_ok(n: int, stride: int) -> bool:
     if stride < 1 or n < 2:
         return False
