@@ -45,7 +45,11 @@ from .complex import ComplexTensor
 
 
 def _grad_on(*ts) -> bool:
-    return torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in ts)
+    if torch.is_grad_enabled():
+        for t in ts:
+            if isinstance(t, torch.Tensor) and t.requires_grad:
+                return True
+    return False
 
 
 def _c(t: torch.Tensor) -> torch.Tensor:

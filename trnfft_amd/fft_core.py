@@ -26,13 +26,26 @@ import torch
 
 from . import _lib
 from .complex import ComplexTensor
-from .dispatch import _require_hip, ptr, stream_handle, target_device, to_device_f32
+from .dispatch import _require_hip, addr, launch, target_device, to_device_f32
 from .plan import FFTAlgorithm, FFTPlan, create_plan, native_plan
 from .precision import _resolve
 
 # n at or below which power-of-two transforms run as a DFT-GEMM (trnfft/fft_core.py:138 uses
 # 256 on NKI); 0 keeps every length on the Stockham kernel.
 _DFT_GEMM_THRESHOLD = 0
+
+
+def _autograd():
+    # (autograd.py imports this module; a plain import statement in every call costs about a microsecond)
+    global _ag_module
+    if _ag_module is None:
+        from . import autograd
+
+        _ag_module = autograd
+    return _ag_module
+
+
+_ag_module = None
 
 
 def fft_core(
@@ -49,8 +62,7 @@ def fft_core(
     if plan is None:
         plan = create_plan(n, inverse=inverse)
     _require_hip("fft_core")
-    from . import autograd as _ag
-
+    _ag = _autograd()
     if plan.algorithm == FFTAlgorithm.COOLEY_TUKEY and n <= _DFT_GEMM_THRESHOLD and not _ag._grad_on(x.real, x.imag):
         return _fft_via_gemm(x, inverse)
     # differentiable when the planes require grad (adjoint on the same kernels)
@@ -73,14 +85,12 @@ def execute_1d(re: torch.Tensor, im: torch.Tensor | None, inverse: bool) -> Comp
     out_re = torch.empty_like(re)
     out_im = torch.empty_like(re)
     ws = None
-    ws_bytes = plan.workspace_bytes(batch)
-    if ws_bytes:
-        ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_execute(
-            plan.handle, batch, ptr(re), ptr(im), ptr(out_re), ptr(out_im), ptr(ws), stream_handle(dev)
-        )
-    _lib.check(rc, "tfa_execute")
+    if plan.may_need_workspace:
+        ws_bytes = plan.workspace_bytes(batch)
+        if ws_bytes:
+            ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=dev)
+    launch("tfa_execute", dev, _lib.lib().tfa_execute, plan.handle, batch, addr(re), addr(im), addr(out_re),
+           addr(out_im), addr(ws))
     out = ComplexTensor._wrap(out_re, out_im)
     return out if out_dev == dev else out.to(out_dev)
 
@@ -108,11 +118,9 @@ def execute_r2c(x: torch.Tensor) -> ComplexTensor:
     batch = x.numel() // n
     plan = native_plan(_lib.KIND_REAL, n, False, dev.index)
     shape = (*x.shape[:-1], n // 2 + 1)
-    out_re = torch.empty(shape, dtype=torch.float32, device=dev)
-    out_im = torch.empty(shape, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_execute(plan.handle, batch, ptr(x), None, ptr(out_re), ptr(out_im), None, stream_handle(dev))
-    _lib.check(rc, "tfa_execute")
+    out_re, out_im = x.new_empty(shape), x.new_empty(shape)
+    launch("tfa_execute", dev, _lib.lib().tfa_execute, plan.handle, batch, addr(x), None, addr(out_re), addr(out_im),
+           None)
     out = ComplexTensor._wrap(out_re, out_im)
     return out if out_dev == dev else out.to(out_dev)
 
@@ -127,10 +135,8 @@ def execute_c2r(re: torch.Tensor, im: torch.Tensor, n: int) -> torch.Tensor:
     im = to_device_f32(im, dev).contiguous()
     batch = re.numel() // (n // 2 + 1)
     plan = native_plan(_lib.KIND_REAL, n, True, dev.index)
-    out = torch.empty((*re.shape[:-1], n), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_execute(plan.handle, batch, ptr(re), ptr(im), ptr(out), None, None, stream_handle(dev))
-    _lib.check(rc, "tfa_execute")
+    out = re.new_empty((*re.shape[:-1], n))
+    launch("tfa_execute", dev, _lib.lib().tfa_execute, plan.handle, batch, addr(re), addr(im), addr(out), None, None)
     return out if out_dev == dev else out.to(out_dev)
 
 
@@ -174,19 +180,16 @@ def execute_strided(re: torch.Tensor, im: torch.Tensor | None, dim: int, inverse
     out_re = torch.empty_like(re)
     out_im = torch.empty_like(re)
     lib = _lib.lib()
-    with torch.cuda.device(dev):
-        nbytes = ctypes.c_size_t(0)
-        _lib.check(lib.tfa_strided_workspace_size(plan.handle, outer, stride, ctypes.byref(nbytes)),
-                   "tfa_strided_workspace_size")
-        if nbytes.value:
-            ws = torch.empty(nbytes.value // 4, dtype=torch.float32, device=dev)
-            rc = lib.tfa_execute_strided_ws(plan.handle, outer, stride, ptr(re), ptr(im), ptr(out_re), ptr(out_im),
-                                            ptr(ws), stream_handle(dev))
-            _lib.check(rc, "tfa_execute_strided_ws")
-        else:
-            rc = lib.tfa_execute_strided(plan.handle, outer, stride, ptr(re), ptr(im), ptr(out_re), ptr(out_im),
-                                         stream_handle(dev))
-            _lib.check(rc, "tfa_execute_strided")
+    nbytes = ctypes.c_size_t(0)
+    _lib.check(lib.tfa_strided_workspace_size(plan.handle, outer, stride, ctypes.byref(nbytes)),
+               "tfa_strided_workspace_size")
+    if nbytes.value:
+        ws = torch.empty(nbytes.value // 4, dtype=torch.float32, device=dev)
+        launch("tfa_execute_strided_ws", dev, lib.tfa_execute_strided_ws, plan.handle, outer, stride, addr(re), addr(im),
+               addr(out_re), addr(out_im), addr(ws))
+    else:
+        launch("tfa_execute_strided", dev, lib.tfa_execute_strided, plan.handle, outer, stride, addr(re), addr(im),
+               addr(out_re), addr(out_im))
     out = ComplexTensor._wrap(out_re, out_im)
     return out if out_dev == dev else out.to(out_dev)
 
@@ -232,11 +235,8 @@ def execute_fft2(re: torch.Tensor, im: torch.Tensor | None, inverse: bool) -> Co
     plan = native_plan(_lib.KIND_FFT2, w, inverse, dev.index, n2=h)
     out_re = torch.empty(re.shape, dtype=torch.float32, device=dev)
     out_im = torch.empty_like(out_re)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_execute(
-            plan.handle, batch, ptr(re), ptr(im), ptr(out_re), ptr(out_im), ptr(None), stream_handle(dev)
-        )
-    _lib.check(rc, "tfa_execute(fft2)")
+    launch("tfa_execute(fft2)", dev, _lib.lib().tfa_execute, plan.handle, batch, addr(re), addr(im), addr(out_re),
+           addr(out_im), None)
     out = ComplexTensor._wrap(out_re, out_im)
     return out if out_dev == dev else out.to(out_dev)
 
@@ -273,11 +273,9 @@ def execute_istft(re: torch.Tensor, im: torch.Tensor, win: torch.Tensor, n_fft: 
     lib = _lib.lib()
     req = -1 if length is None else int(length)
     _lib.check(lib.tfa_istft_length(plan.handle, frames, req, ctypes.byref(out_len)), "tfa_istft_length")
-    out = torch.empty(*lead, out_len.value, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = lib.tfa_istft_execute(plan.handle, batch, frames, ptr(re), ptr(im), ptr(win), ptr(out), req,
-                                   stream_handle(dev))
-    _lib.check(rc, "tfa_istft_execute")
+    out = re.new_empty((*lead, out_len.value))
+    launch("tfa_istft_execute", dev, lib.tfa_istft_execute, plan.handle, batch, frames, addr(re), addr(im), addr(win),
+           addr(out), req)
     return out
 
 
@@ -315,13 +313,9 @@ def execute_stft(x: torch.Tensor, win: torch.Tensor, n_fft: int, hop: int, cente
     for d in lead:
         batch *= d
     shape = (*lead, num_frames, bins) if frames_major else (*lead, bins, num_frames)
-    out_re = torch.empty(*shape, dtype=torch.float32, device=dev)
-    out_im = torch.empty_like(out_re)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_stft_execute(
-            plan.handle, batch, x.shape[-1], ptr(x), ptr(win), ptr(out_re), ptr(out_im), stream_handle(dev)
-        )
-    _lib.check(rc, "tfa_stft_execute")
+    out_re, out_im = x.new_empty(shape), x.new_empty(shape)
+    launch("tfa_stft_execute", dev, _lib.lib().tfa_stft_execute, plan.handle, batch, x.shape[-1], addr(x), addr(win),
+           addr(out_re), addr(out_im))
     if frames_major:
         return out_re.transpose(-2, -1), out_im.transpose(-2, -1)
     return out_re, out_im
@@ -343,13 +337,12 @@ def execute_stft_backward(g_re: torch.Tensor, g_im: torch.Tensor, win: torch.Ten
     plan = native_plan(_lib.KIND_STFT, n_fft, False, dev.index, hop=hop, flags=flags)
     win = win.contiguous()
     b, frames = g_re.shape[0], (g_re.shape[-2] if fm else g_re.shape[-1])
-    out = torch.empty(b, padded_len, dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_stft_backward_execute(plan.handle, b, frames, ptr(g_re), ptr(g_im), ptr(win), ptr(out),
-                                                  padded_len, stream_handle(dev))
-    if rc == _lib.TFA_ERR_UNSUPPORTED:
+    out = g_re.new_empty((b, padded_len))
+    try:
+        launch("tfa_stft_backward_execute", dev, _lib.lib().tfa_stft_backward_execute, plan.handle, b, frames, addr(g_re),
+               addr(g_im), addr(win), addr(out), padded_len)
+    except NotImplementedError:
         return None
-    _lib.check(rc, "tfa_stft_backward_execute")
     return out
 
 
@@ -357,9 +350,7 @@ def execute_fold_edges(d_xp: torch.Tensor, pad: int, length: int) -> None:
     """Adjoint of the reflect padding, in place on the contiguous (b, pad + length + pad) device rows."""
     assert d_xp.is_contiguous() and d_xp.shape[-1] == length + 2 * pad
     dev = d_xp.device
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_stft_fold_edges(d_xp.shape[0], pad, length, ptr(d_xp), stream_handle(dev))
-    _lib.check(rc, "tfa_stft_fold_edges")
+    launch("tfa_stft_fold_edges", dev, _lib.lib().tfa_stft_fold_edges, d_xp.shape[0], pad, length, addr(d_xp))
 
 
 def strided_ok(n: int, stride: int) -> bool:
@@ -382,10 +373,7 @@ def _fft_via_gemm(x: ComplexTensor, inverse: bool) -> ComplexTensor:
     plan = native_plan(_lib.KIND_DFT_GEMM, n, inverse, dev.index)
     out_re = torch.empty_like(re)
     out_im = torch.empty_like(re)
-    with torch.cuda.device(dev):
-        rc = _lib.lib().tfa_execute(
-            plan.handle, batch, ptr(re), ptr(im), ptr(out_re), ptr(out_im), ptr(None), stream_handle(dev)
-        )
-    _lib.check(rc, "tfa_execute(dft_gemm)")
+    launch("tfa_execute(dft_gemm)", dev, _lib.lib().tfa_execute, plan.handle, batch, addr(re), addr(im), addr(out_re),
+           addr(out_im), None)
     out = ComplexTensor._wrap(out_re, out_im)
     return out if out_dev == dev else out.to(out_dev)

@@ -75,7 +75,7 @@ def clear_plan_cache():
 class NativePlan:
     """Owner of one ``tfa_plan`` (device tables) created on a given device."""
 
-    __slots__ = ("handle", "kind", "n", "inverse", "device", "padded_n", "hop", "flags", "n2")
+    __slots__ = ("handle", "kind", "n", "inverse", "device", "padded_n", "hop", "flags", "n2", "may_need_workspace")
 
     def __init__(self, kind: int, n: int, inverse: bool, device: int, hop: int = 0, flags: int = 0, n2: int = 0):
         import torch
@@ -89,6 +89,9 @@ class NativePlan:
             _lib.check(lib.tfa_plan_create(ctypes.byref(handle), ctypes.byref(desc)), "tfa_plan_create")
         self.handle = handle
         self.padded_n = int(lib.tfa_plan_padded_n(handle))
+        # a plan's paths with scratch are taken below some number of rows or at any, so a plan that
+        # needs none for one row never does
+        self.may_need_workspace = self.workspace_bytes(1) > 0
 
     def workspace_bytes(self, batch: int) -> int:
         out = ctypes.c_size_t()
