@@ -204,6 +204,14 @@ int tfa_stft_backward_execute(const tfa_plan* plan, int64_t batch, int64_t n_fra
                               tfa_stream stream);
 
 /*
+ * Rows around a complex transform of real data of any length (trnfft/api.py:38-68): with complete = 0 the first
+ * `half` bins of (batch, n) rows, with complete = 1 the Hermitian rows of length n (half <= n <= 2 half - 1) of
+ * (batch, half) bins, X_k = conj X_{n-k} for k >= half.  Out of place.
+ */
+int tfa_half_rows(int32_t complete, int64_t batch, int64_t n, int64_t half, const float* in_re, const float* in_im,
+                  float* out_re, float* out_im, tfa_stream stream);
+
+/*
  * The reflect padding's adjoint, in place on (batch, pad + length + pad) rows: each kept sample receives the
  * gradient of its mirror images, so that columns [pad, pad + length) are the gradient of the signal
  * (the backward of trnfft/api.py:310-313's F.pad).

@@ -103,3 +103,43 @@ def test_irfft_other_n_keeps_reference_semantics():
         ref = oracle.irfft((re, im), n=n)
         assert got.shape == ref.shape
         torch.testing.assert_close(got.cpu(), ref, atol=1e-5, rtol=1e-4)
+
+
+@pytest.mark.parametrize("n,half", [(2, 2), (3, 2), (5, 3), (6, 4), (7, 5), (100, 51), (101, 51), (90, 51), (51, 51),
+                                    (1000, 501), (1023, 600)])
+@pytest.mark.parametrize("lead", [(1,), (3, 7), (0,)])
+def test_half_rows_are_the_reference_slices_and_completion(n, half, lead):
+    # any n from the number of bins up to twice it less one: bit for bit the composition of slices and flips
+    from trnfft_amd import fft_core
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    re, im = (torch.randn(*lead, half, generator=g, device="cuda") for _ in range(2))
+    full = fft_core.execute_half_rows(re, im, n, half, True)
+    neg = n - half
+    ref_re = torch.cat([re, torch.flip(re[..., 1 : 1 + neg], dims=[-1])], dim=-1)
+    ref_im = torch.cat([im, -torch.flip(im[..., 1 : 1 + neg], dims=[-1])], dim=-1)
+    assert torch.equal(full.real, ref_re) and torch.equal(full.imag, ref_im)
+    part = fft_core.execute_half_rows(full.real, full.imag, n, half, False)
+    assert torch.equal(part.real, re) and torch.equal(part.imag, im)
+
+
+@pytest.mark.parametrize("n,bins", [(622, None), (999, None), (1000, 501), (1001, 501), (900, 501), (501, 501), (400, 201)])
+def test_general_length_rfft_irfft_vs_oracle(n, bins):
+    from conftest import tol_bluestein
+
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(5, n, generator=g)
+    y = trnfft_amd.rfft(x.cuda())
+    assert y.real.is_contiguous() and rel_l2(y.real, y.imag, *oracle.rfft(x)) <= tol_bluestein(n)
+    if bins is not None:
+        re, im = torch.randn(5, bins, generator=g), torch.randn(5, bins, generator=g)
+        got = trnfft_amd.irfft(ComplexTensor(re.cuda(), im.cuda()), n=n)
+        ref = oracle.irfft((re, im), n=n)
+        assert got.shape == ref.shape
+        assert rel_l2(got, torch.zeros_like(got), ref, torch.zeros_like(ref)) <= tol_bluestein(n)
+
+
+def test_irfft_past_the_completed_length_is_refused_as_before():
+    s = ComplexTensor(torch.randn(2, 5).cuda(), torch.randn(2, 5).cuda())
+    with pytest.raises(RuntimeError):
+        trnfft_amd.irfft(s, n=12)  # the completion has 9 elements at most

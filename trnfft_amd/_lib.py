@@ -49,6 +49,7 @@ EXPORTS = (
     "tfa_istft_execute",
     "tfa_stft_backward_execute",
     "tfa_stft_fold_edges",
+    "tfa_half_rows",
     "tfa_complex_gemm",
     "tfa_complex_gemm_ex",
     "tfa_complex_gemm_batched",
@@ -107,6 +108,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tfa_stft_backward_execute.restype = ctypes.c_int
     lib.tfa_stft_fold_edges.argtypes = [_i64, _i64, _i64, _vp, _vp]
     lib.tfa_stft_fold_edges.restype = ctypes.c_int
+    lib.tfa_half_rows.argtypes = [_i32, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp]
+    lib.tfa_half_rows.restype = ctypes.c_int
     lib.tfa_complex_gemm.argtypes = [_i64, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp, _i64, _vp]
     lib.tfa_complex_gemm.restype = ctypes.c_int
     lib.tfa_complex_gemm_ex.argtypes = [_i64, _i64, _i64, _vp, _vp, _i64, _i32, _vp, _vp, _i64, _i32, ctypes.c_float,

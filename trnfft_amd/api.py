@@ -68,6 +68,9 @@ def rfft(input: torch.Tensor, n: int | None = None) -> ComplexTensor:
         return _ag.r2c(input)
     result = _real_1d(input, inverse=False)
     half = n // 2 + 1
+    if (result.real.is_cuda and result.real.dtype == torch.float32 and result.real.numel() > n  # (one row: a view)
+            and not _ag._grad_on(result.real, result.imag)):
+        return _fc.execute_half_rows(result.real, result.imag, n, half, False)
     return ComplexTensor(result.real[..., :half], result.imag[..., :half])
 
 
@@ -79,6 +82,14 @@ def irfft(input: ComplexTensor, n: int | None = None) -> torch.Tensor:
         _resolve(None)
         _require_hip("irfft")
         return _ag.c2r(input.real, input.imag, n)
+    re, im = input.real, input.imag
+    half = re.shape[-1]
+    if (re.is_cuda and re.dtype == torch.float32 == im.dtype and 1 <= half <= n <= 2 * half - 1 and n > 1
+            and not _ag._grad_on(re, im)):
+        # completion and inverse transform, one launch each
+        _resolve(None)
+        _require_hip("irfft")
+        return fft_core(_fc.execute_half_rows(re, im, n, half, True), inverse=True).real
     dev = input.real.device
     full_re = torch.zeros(*input.shape[:-1], n, dtype=input.dtype, device=dev)
     full_im = torch.zeros(*input.shape[:-1], n, dtype=input.dtype, device=dev)

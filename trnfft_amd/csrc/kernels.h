@@ -308,6 +308,11 @@ struct RealArgs {
 };
 hipError_t launch_real(int n, const RealArgs& a);
 
+// (batch, n) complex rows -> their first `half` bins, or (batch, half) bins -> Hermitian (batch, n) rows (complete;
+// half <= n <= 2 * half - 1)
+hipError_t launch_half_rows(bool complete, const float* in_re, const float* in_im, float* out_re, float* out_im,
+                            long long batch, int n, int half, hipStream_t stream);
+
 struct IstftArgs {
   const float* spec_re;  // (batch, bins, n_frames), bins = n_fft/2+1 (n_fft when two_sided)
   const float* spec_im;

@@ -1123,6 +1123,19 @@ int tfa_stft_backward_execute(const tfa_plan* plan, int64_t batch, int64_t n_fra
   return e == hipSuccess ? TFA_OK : hip_fail(e, "stft backward launch");
 }
 
+int tfa_half_rows(int32_t complete, int64_t batch, int64_t n, int64_t half, const float* in_re, const float* in_im,
+                  float* out_re, float* out_im, tfa_stream stream) {
+  if (batch < 0 || half < 1 || half > n) return fail(TFA_ERR_INVALID, "need 1 <= half <= n");
+  if (complete && n > 2 * half - 1) return fail(TFA_ERR_INVALID, "n is longer than the bins complete");
+  if (n > INT32_MAX) return fail(TFA_ERR_UNSUPPORTED, "row too long");
+  if (batch == 0) return TFA_OK;
+  if (!in_re || !in_im || !out_re || !out_im) return fail(TFA_ERR_INVALID, "null data pointer");
+  hipError_t e = tfa::launch_half_rows(complete != 0, in_re, in_im, out_re, out_im, batch, (int)n, (int)half,
+                                       static_cast<hipStream_t>(stream));
+  if (e == hipErrorInvalidValue) return fail(TFA_ERR_UNSUPPORTED, "rows beyond the launch grid");
+  return e == hipSuccess ? TFA_OK : hip_fail(e, "half rows launch");
+}
+
 int tfa_stft_fold_edges(int64_t batch, int64_t pad, int64_t length, float* grad_padded, tfa_stream stream) {
   if (batch < 0 || pad < 0 || length < 1) return fail(TFA_ERR_INVALID, "bad dimension");
   if (pad >= length) return fail(TFA_ERR_INVALID, "reflect padding needs more samples than pad");

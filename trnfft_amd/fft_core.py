@@ -140,6 +140,17 @@ def execute_c2r(re: torch.Tensor, im: torch.Tensor, n: int) -> torch.Tensor:
     return out if out_dev == dev else out.to(out_dev)
 
 
+def execute_half_rows(re: torch.Tensor, im: torch.Tensor, n: int, half: int, complete: bool) -> ComplexTensor:
+    """The first `half` bins of (..., n) device rows, or (complete) the Hermitian (..., n) rows of (..., half)
+    bins, half <= n <= 2 * half - 1 (the slices and the completion of trnfft/api.py:44-46, 55-66)."""
+    re, im = re.contiguous(), im.contiguous()
+    shape = (*re.shape[:-1], n if complete else half)
+    out_re, out_im = re.new_empty(shape), re.new_empty(shape)
+    launch("tfa_half_rows", re.device, _lib.lib().tfa_half_rows, int(complete), re.numel() // re.shape[-1], n, half,
+           addr(re), addr(im), addr(out_re), addr(out_im))
+    return ComplexTensor._wrap(out_re, out_im)
+
+
 # longest power-of-two axis the single-pass strided kernel transforms in place of a transpose
 # round trip, longest other axis (Bluestein padded length m <= 4096), and the strided multi-pass
 # path's reach (longer power-of-two axes: two passes with >= 4 trailing columns, three passes from
