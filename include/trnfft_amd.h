@@ -263,6 +263,15 @@ int tfa_complex_gemm_ws(int64_t batch, int64_t m, int64_t n, int64_t k, const fl
                         int64_t stride_b, int32_t b_op, float alpha, const float* bias_re, const float* bias_im,
                         float* c_re, float* c_im, int64_t ldc, int64_t stride_c, void* workspace, tfa_stream stream);
 
+/*
+ * Sums over the rows of two row-major (rows, cols) planes (the bias gradient of
+ * trnfft/nki/autograd.py:125-155).  `workspace`: tfa_column_sums_workspace_size bytes of device memory (NULL: the rows
+ * are summed by one workgroup per 64 columns).
+ */
+int tfa_column_sums_workspace_size(int64_t rows, int64_t cols, size_t* bytes);
+int tfa_column_sums(int64_t rows, int64_t cols, const float* re, const float* im, float* out_re, float* out_im,
+                    void* workspace, tfa_stream stream);
+
 /* Thread-local message describing the last failure on this thread ("" if none). */
 const char* tfa_last_error(void);
 

@@ -272,3 +272,15 @@ def test_gemm_nonfinite_operands(k):
         assert torch.equal(torch.isneginf(x), torch.isneginf(y))
     ok = [torch.isfinite(y) for y in ref]
     assert rel_l2(got.real[ok[0]], got.imag[ok[1]], ref[0][ok[0]], ref[1][ok[1]]) <= _tol_k(k)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 65), (33, 64), (63, 130), (64, 1), (1000, 257), (8192, 1024), (100000, 3)])
+def test_column_sums_vs_float64(rows, cols):
+    from trnfft_amd.dispatch import column_sums
+
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    re, im = (torch.randn(rows, cols, generator=g, device="cuda") for _ in range(2))
+    got = column_sums(re, im)
+    # chains of at most rows / 32 additions between pairwise ones; sqrt of that many roundings of 2^-24
+    tol = 2.0**-24 * (4 + math.sqrt(rows / 32 + 1))
+    assert rel_l2(*got, re.double().sum(0), im.double().sum(0)) <= tol

@@ -55,6 +55,8 @@ EXPORTS = (
     "tfa_complex_gemm_batched",
     "tfa_complex_gemm_workspace_size",
     "tfa_complex_gemm_ws",
+    "tfa_column_sums_workspace_size",
+    "tfa_column_sums",
     "tfa_last_error",
     "tfa_abi_version",
 )
@@ -123,6 +125,10 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tfa_complex_gemm_ws.argtypes = [_i64, _i64, _i64, _i64, _vp, _vp, _i64, _i64, _i32, _vp, _vp, _i64, _i64,
                                         _i32, ctypes.c_float, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp]
     lib.tfa_complex_gemm_ws.restype = ctypes.c_int
+    lib.tfa_column_sums_workspace_size.argtypes = [_i64, _i64, ctypes.POINTER(ctypes.c_size_t)]
+    lib.tfa_column_sums_workspace_size.restype = ctypes.c_int
+    lib.tfa_column_sums.argtypes = [_i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp]
+    lib.tfa_column_sums.restype = ctypes.c_int
     lib.tfa_execute_noalloc.argtypes = [_vp, _i64, _vp, _vp, _vp, _vp, _vp]
     lib.tfa_execute_noalloc.restype = ctypes.c_int
     lib.tfa_last_error.argtypes = []

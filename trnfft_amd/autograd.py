@@ -484,7 +484,7 @@ class _ComplexGEMMFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_re, g_im):
-        from .dispatch import gemm_ex
+        from .dispatch import column_sums, gemm_ex
 
         a_re, a_im, b_re, b_im = ctx.saved_tensors
         need = ctx.needs_input_grad
@@ -512,7 +512,7 @@ class _ComplexGEMMFn(torch.autograd.Function):
             else:
                 db_re, db_im = gemm_ex(a_re, a_im, _lib.OP_C, g_re, g_im, _lib.OP_N, what="complex_gemm backward dB")
         if ctx.has_bias and (need[4] or need[5]):
-            dbias_re, dbias_im = g_re.sum(0), g_im.sum(0)
+            dbias_re, dbias_im = column_sums(g_re, g_im) if g_re.numel() else (g_re.sum(0), g_im.sum(0))
         return da_re, da_im, db_re, db_im, dbias_re, dbias_im, None, None
 
 

