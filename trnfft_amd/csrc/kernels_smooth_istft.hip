@@ -7,25 +7,30 @@
 // values are the frame's samples in pairs; then every owned sample sums its frames from LDS.
 //
 // Bound by the latencies between its barriers, as the forward kernel: 64 x 201 x 1001 bins at n_fft 400, hop 160,
-// in 61 us, against 306 for one 1024-point Bluestein chain per frame.  With the bins staged four loads at a
+// in 59 us, against 306 for one 1024-point Bluestein chain per frame.  With the bins staged four loads at a
 // time and a division per sample 121 us; every load issued before the first store, and a thread keeping one phase of
-// the hop with its window values, 88; two workgroups per CU (smooth_lds) 61.
+// the hop with its window values, 88; two workgroups per CU (smooth_lds) 61, three 59.
 #include "smooth.h"
 
 namespace tfa {
 
 // Frames per workgroup: above the longest halo that the plan accepts (32 frames up to n_fft 128, else 16)
-__host__ __device__ constexpr int smooth_istft_frames(int n) { return n <= 128 ? 64 : n <= 448 ? 32 : 20; }
+template <int N>
+constexpr int smooth_istft_frames() {
+  return N <= 128 ? 64 : N <= 448 ? 32 : 20;
+}
+template <int N>
+using IstftSmooth = Smooth<N / 2, smooth_pad<N / 2, smooth_istft_frames<N>()>(4 * N)>;
 
 template <int N>
-__global__ __launch_bounds__((SmoothGroup<N / 2, smooth_istft_frames(N)>::THREADS)) void istft_smooth_kernel(
+__global__ __launch_bounds__((SmoothGroup<N / 2, smooth_istft_frames<N>()>::THREADS)) void istft_smooth_kernel(
     const float* __restrict__ sre, const float* __restrict__ sim, const float* __restrict__ win,
     float* __restrict__ out, const float2* __restrict__ tw, const float2* __restrict__ twn, int n_frames, int hop,
     int halo, int owned, int tiles_per_signal, int expected_len, int start, int write_len, int out_pitch, float scale,
     bool adjoint, bool frames_major) {
-  constexpr int H = N / 2, K = H + 1, FR = smooth_istft_frames(N);
+  constexpr int H = N / 2, K = H + 1, FR = smooth_istft_frames<N>();
   using G = SmoothGroup<H, FR>;
-  using S = Smooth<H>;
+  using S = IstftSmooth<N>;
   constexpr int N1 = S::N1, N2 = S::N2, AREA = S::AREA, THREADS = G::THREADS;
   float2* const lds = smooth_lds;  // FR * AREA
   float* const wl = reinterpret_cast<float*>(lds + FR * AREA);  // the window, N floats
@@ -188,8 +193,8 @@ __global__ __launch_bounds__((SmoothGroup<N / 2, smooth_istft_frames(N)>::THREAD
 hipError_t launch_istft_smooth(int n_fft, const IstftArgs& a) {
   hipError_t e = hipErrorInvalidValue;
   smooth_dispatch(n_fft, [&](auto n) {
-    constexpr int N = decltype(n)::value, FR = smooth_istft_frames(N);
-    constexpr unsigned LDS = (FR * Smooth<N / 2>::AREA + N / 2) * 8;
+    constexpr int N = decltype(n)::value, FR = smooth_istft_frames<N>();
+    constexpr unsigned LDS = (FR * IstftSmooth<N>::AREA + N / 2) * 8;
     static_assert(LDS <= kSmoothLds, "frame tile exceeds LDS");
     const int owned = FR - a.halo;
     if (a.halo < 0 || a.hop < 1 || owned < 1) return;

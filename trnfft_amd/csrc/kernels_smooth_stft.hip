@@ -5,18 +5,24 @@
 // (Z_k + conj Z_{H-k}) / 2 - i W_N^k (Z_k - conj Z_{H-k}) / 2.  (Two frames in one transform would save nothing
 // here and let a non-finite sample reach a frame that does not hold it.)
 //
-// Bound by the latencies between its four barriers, at 1.5 to 3 workgroups per CU, and by the bin rows' partial
-// lines: 64 x 160000 at n_fft 400, hop 160 (144 MB) in 59 us, against 148 for one 768-point Bluestein chain
+// Bound by the latencies between its four barriers, at two or three workgroups per CU, and by the bin rows' partial
+// lines: 64 x 160000 at n_fft 400, hop 160 (144 MB) in 51 us, against 148 for one 768-point Bluestein chain
 // per frame.  Samples read from memory frame by frame instead of as the tile's span, with the window and the
 // twiddles read again in each round, kept the L1 busy (27 accesses per load instruction): 75 us.
 #include "smooth.h"
 
 namespace tfa {
 
-// Frames per workgroup: their bins leave in runs of that many floats, and their areas fit kSmoothLds.  Calls of
-// few frames take a quarter, so that four times the workgroups share the work of a tile: 1 x 16000 at n_fft
-// 400, hop 400, 14.7 -> 8.7 us.
-__host__ __device__ constexpr int smooth_stft_frames(int n) { return n <= 128 ? 64 : n <= 448 ? 32 : 16; }
+// Frames per workgroup: their bins leave in runs of that many floats (20 and 26, which would let another
+// workgroup share the CU, took 12 to 20 % longer than 16).  Calls of few frames take a quarter, so that four times the
+// workgroups share the work of a tile: 1 x 16000 at n_fft 400, hop 400, 14.7 -> 8.7 us.
+template <int N>
+constexpr int smooth_stft_frames() {
+  return N <= 128 ? 64 : N <= 448 ? 32 : 16;
+}
+// (n_fft 400: three workgroups per CU instead of two, 59 -> 51 us)
+template <int N, int FR>
+using StftSmooth = Smooth<N / 2, smooth_pad<N / 2, FR>(0)>;
 
 template <int N, int FR>
 __global__ __launch_bounds__((SmoothGroup<N / 2, FR>::THREADS)) void stft_smooth_kernel(
@@ -25,7 +31,7 @@ __global__ __launch_bounds__((SmoothGroup<N / 2, FR>::THREADS)) void stft_smooth
     int pad, int n_frames, int n_bins, int tiles_per_signal, float scale, bool frames_major) {
   constexpr int H = N / 2;
   using G = SmoothGroup<H, FR>;
-  using S = Smooth<H>;
+  using S = StftSmooth<N, FR>;
   constexpr int N1 = S::N1, N2 = S::N2, AREA = S::AREA, THREADS = G::THREADS;
   float2* const lds = smooth_lds;  // FR * AREA
   const unsigned tile = xcd_tile_remap32(blockIdx.x, gridDim.x);
@@ -165,15 +171,14 @@ __global__ __launch_bounds__((SmoothGroup<N / 2, FR>::THREADS)) void stft_smooth
     }
     return;
   }
+  constexpr int KS = THREADS / FR, KN = H / 2 + 1;  // bin pairs per step, of KN
   const int fr = t % FR;
-  if (f0 + fr >= n_frames) return;
+  if (f0 + fr >= n_frames || t >= KS * FR) return;
   const float2* Z = lds + fr * AREA;
   // 32-bit offsets from the signal's (uniform) base: the host keeps n_bins * n_frames within 2^30
   const size_t ob = (size_t)b * n_bins * n_frames + f0;
   float* ore = out_re + ob;
   float* oim = out_im + ob;
-  constexpr int KS = THREADS / FR, KN = H / 2 + 1;  // bin pairs per step, of KN
-  static_assert(THREADS % FR == 0, "whole steps");
   const bool two_sided = n_bins == N;
   const auto put = [&](int k, float2 y) {
     const unsigned off = (unsigned)(fr + k * n_frames);
@@ -204,7 +209,7 @@ __global__ __launch_bounds__((SmoothGroup<N / 2, FR>::THREADS)) void stft_smooth
 
 template <int N, int FR>
 static hipError_t launch_stft_tiles(const StftArgs& a) {
-  constexpr unsigned LDS = FR * Smooth<N / 2>::AREA * 8;
+  constexpr unsigned LDS = FR * StftSmooth<N, FR>::AREA * 8;
   static_assert(LDS <= kSmoothLds, "frame tile exceeds LDS");
   const int tiles = (a.n_frames + FR - 1) / FR;
   const long long blocks = a.batch * (long long)tiles;
@@ -218,7 +223,7 @@ static hipError_t launch_stft_tiles(const StftArgs& a) {
 hipError_t launch_stft_smooth(int n_fft, const StftArgs& a) {
   hipError_t e = hipErrorInvalidValue;
   smooth_dispatch(n_fft, [&](auto n) {
-    constexpr int N = decltype(n)::value, FR = smooth_stft_frames(N);
+    constexpr int N = decltype(n)::value, FR = smooth_stft_frames<N>();
     e = a.batch * (long long)((a.n_frames + FR - 1) / FR) >= kNumCUs ? launch_stft_tiles<N, FR>(a)
                                                                     : launch_stft_tiles<N, FR / 4>(a);
   });

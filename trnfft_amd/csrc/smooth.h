@@ -88,11 +88,12 @@ template <int DIR> struct Dft<30, DIR> : DftSplit<5, 6, DIR> {};
 // Forward transform of N points, one LDS area of AREA float2 per transform.  Item j2 < N2 of the first pass
 // holds x[j2 + N2 j1] (j1 < N1), item k1 < N1 of the second holds X[k1 + N1 k2] (k2 < N2).  The exchange
 // has an odd pitch, and so has the area, so that both passes and lanes over several transforms at
-// one index meet distinct banks.  (The inverse is the forward transform with re and im exchanged in both
+// one index meet distinct banks.  (PAD false: a pitch of N2, where that lets another workgroup share the CU; 100-point
+// rows are 14 % slower without the padding.)  (The inverse is the forward transform with re and im exchanged in both
 // its input and its output.)
-template <int N>
+template <int N, bool PAD = true>
 struct Smooth {
-  static constexpr int N1 = smooth_n1(N), N2 = N / N1, PITCH = N2 | 1;
+  static constexpr int N1 = smooth_n1(N), N2 = N / N1, PITCH = PAD ? N2 | 1 : N2;
   static constexpr int AREA = (N1 * PITCH > N + 1 ? N1 * PITCH : N + 1) | 1;
 
   // tw: W_N^(k1 j2) at k1 * N2 + j2
@@ -121,6 +122,14 @@ struct SmoothGroup {
   static constexpr int THREADS = (XF * WIDE + 63) / 64 * 64;
   static constexpr int ROUNDS = (XF * S::N2 + THREADS - 1) / THREADS;
 };
+
+constexpr int kSmoothLds3 = 53760;  // LDS that lets three workgroups share a CU (160 KB in units of 1280 bytes)
+// Whether XF areas of N points, and `more` bytes, take three workgroups per CU only without padding
+template <int N, int XF>
+constexpr bool smooth_pad(int more) {
+  return !(XF * Smooth<N, true>::AREA * 8 + more > kSmoothLds3 && XF * Smooth<N, false>::AREA * 8 + more <= kSmoothLds3 &&
+           Smooth<N>::N2 % 8 != 0);
+}
 
 // The kernels' LDS.  Its size is given at the launch: where the compiler knows that LDS leaves room for few
 // waves it rounds the register count up to just that many per SIMD, and a workgroup of 5 waves, which
