@@ -33,6 +33,7 @@ import torch
 ROOT = os.path.dirname(os.path.abspath(__file__))
 HBM_PEAK = 8.0e12  # MI355X HBM3E, bytes/s
 FP32_PEAK = 157.3e12  # MI355X dense fp32 (matrix), flop/s
+BF16_PEAK = 2.5e15  # MI355X dense bf16 (matrix), flop/s
 
 
 def make_c2c_input(batch: int, n: int, seed: int = 42):
@@ -368,7 +369,9 @@ def bench_secondary():
         if kind == "hbm":
             r["frac_hbm"] = round(nbytes / t / HBM_PEAK, 4)
         else:
+            # fp32 products run as six bf16 products each, so the rate may pass the fp32 matrix peak
             r["frac_fp32_mfma"] = round(flops / t / FP32_PEAK, 4)
+            r["frac_bf16_mfma_issued"] = round(6 * flops / t / BF16_PEAK, 4)
         if sets is not None:
             r["buffer_sets"] = sets
         if note:
@@ -406,8 +409,7 @@ def bench_secondary():
             note="inverse of c2: spectra " + ("(64, 257, 626), the reference's layout" if not tag else
                                               "(64, 626, 257)") + " in, 64 x 160000 samples out")
     del specs, ys
-    # C2's signals at n_fft 400 (25 ms at 16 kHz), hop 160: one Bluestein chain per frame (the
-    # reference's layout)
+    # C2's signals at n_fft 400 (25 ms at 16 kHz), hop 160 (the reference's layout)
     w400 = torch.hann_window(400).to(dev)
     p400 = native_plan(_lib.KIND_STFT, 400, False, dev.index, hop=160, flags=bm)
     frames = 1 + 160000 // 160
@@ -415,15 +417,14 @@ def bench_secondary():
     os_ = [(torch.empty(64, 201, frames, device=dev), torch.empty(64, 201, frames, device=dev)) for _ in range(S)]
     t = _time_rot(lambda k, st: chk(L.tfa_stft_execute(p400.handle, 64, 160000, P(xs[k]), P(w400), P(os_[k][0]),
                                                    P(os_[k][1]), st)), S)
-    rec("stft_64x160000_nfft400", t, 64 * frames * 2 * 5 * 768 * math.log2(768), nbytes, sets=S,
-        note="non-power-of-two n_fft: two 768-point transforms per frame (gflops counts those), VALU-bound")
-    # its inverse: one inverse Bluestein chain per frame (1024 points: every sample is kept)
+    rec("stft_64x160000_nfft400", t, flops_fft(400, 64 * frames) / 2, nbytes, sets=S,
+        note="non-power-of-two n_fft, direct 200-point transform per real frame; flops = 2.5 N log2 N per frame")
     ip400 = native_plan(_lib.KIND_STFT, 400, True, dev.index, hop=160, flags=bm)
     ys = [torch.empty(64, 160000, device=dev) for _ in range(S)]
     t = _time_rot(lambda k, st: chk(L.tfa_istft_execute(ip400.handle, 64, frames, P(os_[k][0]), P(os_[k][1]),
                                                         P(w400), P(ys[k]), 160000, st)), S)
-    rec("istft_64x201x1001_nfft400", t, 64 * frames * 2 * 5 * 1024 * 10, nbytes, sets=S,
-        note="inverse of the n_fft 400 line: two 1024-point transforms per frame (gflops counts those), VALU-bound")
+    rec("istft_64x201x1001_nfft400", t, flops_fft(400, 64 * frames) / 2, nbytes, sets=S,
+        note="inverse of the n_fft 400 line; flops = 2.5 N log2 N per frame")
     del xs, os_, ys
     # C3: Bluestein (fused, one launch)
     for n, b in [(1000, 1024), (4099, 256)]:
