@@ -305,7 +305,8 @@ def stft(
 
     Power-of-two n_fft in [16, 4096], and other n_fft from 9 to 2731 (2048 two-sided), run as
     one fused kernel that reads the raw waveform (framing, padding, window, transform -- one
-    Bluestein chain per frame for non-power-of-two n_fft -- and the (freq, time) transpose in one
+    direct transform per frame for n_fft 36 to 640 that are multiples of 4 without a prime factor
+    above 7, one Bluestein chain per frame for the rest -- and the (freq, time) transpose in one
     pass); with a pad_mode other than "reflect" the signal is padded on the device first (the
     reference's F.pad) and the fused kernel frames the padded signal.  Other n_fft keep the
     reference's composition on the device: pad, frame gather, window, then the transform kernels
@@ -388,7 +389,7 @@ def istft(
     """Inverse STFT by overlap-add with window-sum normalisation (trnfft/api.py:368-470).
 
     One fused kernel (completion, inverse transform -- two frames per transform for power-of-two
-    n_fft in [16, 4096], onesided or two-sided spectra; one inverse Bluestein chain per frame for
+    n_fft in [16, 4096], onesided or two-sided spectra; one direct or Bluestein transform per frame for
     other n_fft in [9, 2048], onesided -- window, overlap-add, envelope division, trim), whose
     spectra gradient at power-of-two n_fft is the fused forward STFT of the envelope-divided
     gradient; for window gradients, gradients at other n_fft, two-sided spectra at other n_fft or
@@ -459,7 +460,7 @@ def _istft_fused(spec, n_fft, hop, win_length, window, center, normalized, onesi
 
     re, im = spec.real, spec.imag
     # power-of-two n_fft in [16, 4096] (two frames per inverse transform; onesided or two-sided
-    # spectra), other n_fft in [9, 2048] (one inverse Bluestein chain per frame, onesided)
+    # spectra), other n_fft in [9, 2048] (one direct or Bluestein transform per frame, onesided)
     pow2 = n_fft & (n_fft - 1) == 0
     bins = n_fft // 2 + 1 if onesided else n_fft
     if ((not onesided and not pow2) or (pow2 and not 16 <= n_fft <= 4096) or (not pow2 and not 9 <= n_fft <= 2048)

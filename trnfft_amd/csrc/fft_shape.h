@@ -208,7 +208,8 @@ __host__ __device__ constexpr int stft_blue_nmax(int m) {
 // samples, hop 2n/5, every E in {4..32} dividing m and 2..64 frames per workgroup; the kernel is
 // VALU-bound, ~1 wavefront-instruction per 64 points per pass): n_fft 30 (m 64) 128 us, 100 (192)
 // 148, 200 (384) 177, 257 (512) 177, 400 (768) 186, 600 (1024) 188, 1000 (1536) 199, 1300 (2048)
-// 187, 2000 (3072) 232.  (m = 1024 at E = 16 / 16 frames, the first shape: 270 us for n_fft 400;
+// 187, 2000 (3072) 232.  (Measured before smooth lengths, n_fft 400
+// among them, had kernels of their own.  m = 1024 at E = 16 / 16 frames, the first shape: 270 us for n_fft 400;
 // the shortest-length rule with the truncated filter took n_fft 400 from 1024 to 768 points,
 // 320 from 1024 to 512 and 600 from 2048 to 1024.)
 __host__ __device__ constexpr int stft_blue_epth(int m) {
@@ -226,7 +227,7 @@ __host__ __device__ constexpr int stft_blue_area(int m, int frames) {
   while (a % 64 != g) a += 4;
   return a;
 }
-// Inverse STFT at n_fft that is not a power of two (one inverse Bluestein chain per frame, m >=
+// Inverse STFT at n_fft that is neither a power of two nor smooth (one inverse Bluestein chain per frame, m >=
 // 2n - 1 since every sample of a frame is kept): elements per thread and frames per workgroup
 // (owned frames + the recomputed halo of floor((n-1)/hop) frames; up to 1024 threads within the
 // LDS, which also holds the window).  Measured on MI355X (64 signals, 160000 output samples):

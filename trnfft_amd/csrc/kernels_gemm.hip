@@ -10,16 +10,18 @@
 // Against 64 bits (random normal operands, relative 2-norm) that is closer than fp32 products were: 1.7e-7
 // against 8.1e-7 at K = 1024, 8e-8 against 1.45e-7 at K = 33.  The matrix rate is what pays for it: 8192 x
 // 1024 x 1024 takes 325 us back to back (515 with v_mfma_f32_32x32x2f32 at 85 % of its peak), 412 GF of bf16
-// products at 1.27 PF; the matrix cores are busy 68 % of the cycles, at the 1.66 GHz that the card then
-// runs at (rocprofv3; the same work spread thinner clocked higher: 52 % busy, 1.95 GHz, 10 % slower).
+// products at 1.27 PF; the matrix cores are busy 67 to 68 % of the cycles, at 1.66 to 1.83 GHz by card
+// (rocprofv3; spread thinner, 52 % busy, it clocked 1.95 GHz and took 390 us against 348), probably the power limit.
+// Where one product dominates a sum (operands like exp(6 N(0, 1))) its truncated bits show: up to 1.4e-7.
 //
 // One kernel computes all four real products: each k-step loads the fragments of the three pieces of
 // A_re/A_im and B_re/B_im once from LDS for 24 MFMAs per 32 x 32 tile of the two accumulator sets (the
 // NKI kernel's "stationary reuse" idea, trnfft/nki/dispatch.py:121-200 and :267-345, in CDNA4 form).
 // Workgroup tile 128 x 128 (per plane), 8 waves of 64 x 32, 16 k per stage, two stages in LDS (one
 // barrier per stage): while one stage is multiplied the next is split and stored, and the one after
-// it is on its way from memory in registers.  Waves w and w + 4 share a SIMD; one of them splits before
-// its MFMAs and the other after, so that the matrix core has work throughout.
+// it is on its way from memory in registers.  The splitting, and the fp32 additions of the stage before, are
+// pinned behind the MFMA pairs that hide them (splitting before or after the MFMAs by wave: 1109 to 1190 us
+// for the linear layer's three products, 1030 pinned).
 #include <algorithm>
 #include <utility>
 

@@ -8,7 +8,7 @@
 // Bound by the latencies between its four barriers, at two or three workgroups per CU, and by the bin rows' partial
 // lines: 64 x 160000 at n_fft 400, hop 160 (144 MB) in 51 us, against 148 for one 768-point Bluestein chain
 // per frame.  Samples read from memory frame by frame instead of as the tile's span, with the window and the
-// twiddles read again in each round, kept the L1 busy (27 accesses per load instruction): 75 us.
+// twiddles read again in each round, kept the L1 busy (28.0 M accesses for 1.35 M memory instructions): 75 us.
 #include "smooth.h"
 
 namespace tfa {

@@ -1,4 +1,5 @@
-// Fused STFT and inverse STFT for n_fft that is not a power of two: one Bluestein chain per frame
+// Fused STFT and inverse STFT for n_fft that is neither a power of two nor a smooth length (smooth.h): one Bluestein
+// chain per frame
 // (framing, padding, window and the (freq, time) layout fused in the forward kernel; completion,
 // window, overlap-add and envelope in the inverse kernel).
 #include "kernels.h"
@@ -18,7 +19,7 @@ namespace tfa {
 // M only has to hold the linear convolution for the kept bins: output k < n_bins sums
 // y[j] h[k - j] over j < n, i.e. the filter taps -(n-1) .. n_bins-1, so with only those taps in the
 // filter (the plan's) any M >= n + n_bins - 1 gives the reference's values without wrap-around,
-// and M is the shortest power of two or 3 * 2^k that does (768 for n_fft = 400 onesided, against
+// and M is the shortest power of two or 3 * 2^k that does (768 for n_fft = 441 onesided, against
 // the reference's 1024).  The samples are the elements e < EIN of each thread and the kept bins
 // (n_bins <= M/2) the elements e < E/2.
 template <int M, int E, int FR>
