@@ -284,3 +284,23 @@ def test_column_sums_vs_float64(rows, cols):
     # chains of at most rows / 32 additions between pairwise ones; sqrt of that many roundings of 2^-24
     tol = 2.0**-24 * (4 + math.sqrt(rows / 32 + 1))
     assert rel_l2(*got, re.double().sum(0), im.double().sum(0)) <= tol
+
+
+@pytest.mark.parametrize("k", [1, 40])
+@pytest.mark.parametrize("value", [1 + 2.0**-7 - 2.0**-23, 1 + 2.0**-8 - 2.0**-16, 2 - 2.0**-23, None])
+def test_gemm_sums_of_one_product(k, value):
+    # every sum is one product (one nonzero k per row), element by element.  What the bf16 pieces leave out is at
+    # most 2 * 2^-24 of the operands' powers of two, and the sum is rounded at its full size once (2^-23 where
+    # that is a truncation): 2^-22 of the product
+    g = torch.Generator(device="cuda").manual_seed(7)
+    m, n = 130, 140
+    a, b = torch.zeros(m, k, device="cuda"), torch.zeros(k, n, device="cuda")
+    rows = torch.arange(m, device="cuda")
+    draw = lambda *s: torch.rand(*s, generator=g, device="cuda") + 0.5 if value is None else torch.full(s, value, device="cuda")  # noqa: E731
+    a[rows, rows % k] = draw(m)
+    b[:] = draw(k, n)
+    got = trnfft_amd.complex_matmul(ComplexTensor(a, torch.zeros_like(a)), ComplexTensor(b, b))
+    ref = a.double() @ b.double()
+    for plane in (got.real, got.imag):
+        err = (plane.double() - ref) / ref
+        assert err.abs().max() <= 2.0**-22

@@ -3,16 +3,21 @@
 //   C = alpha * (op(A) @ op(B)) + bias,  op(X) = X, X^T, conj(X)^T or conj(X)
 //   C_re = A_re B_re - A_im B_im,  C_im = A_re B_im + A_im B_re   (on the op'ed operands)
 //
-// Every fp32 operand is the exact sum of three bf16 pieces of 8 significant bits each (x1 = the top
-// 16 bits of x, x2 = those of x - x1, x3 = x - x1 - x2), so a product a b is the sum of nine bf16
-// products, each exact in fp32; the six of a weight of 2^-16 or more (a1 b1, a1 b2, a2 b1, a2 b2, a1 b3,
-// a3 b1) run on the matrix cores into fp32 accumulators, the other three are below 2^-24 of a b.
-// Against 64 bits (random normal operands, relative 2-norm) that is closer than fp32 products were: 1.7e-7
-// against 8.1e-7 at K = 1024, 8e-8 against 1.45e-7 at K = 33.  The matrix rate is what pays for it: 8192 x
+// Every fp32 operand is the exact sum of three bf16 pieces of 8 significant bits each, every one rounded to
+// nearest (x1 = bf16(x), x2 = bf16(x - x1), x3 = x - x1 - x2; Henry, Tang and Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", ARITH 2019), so a product a b is the sum
+// of nine bf16 products, each exact in fp32.  Six of them (a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1) run on the
+// matrix cores into fp32 accumulators.  x2 is at most 2^-8 and x3 2^-16 of the power of two below |x|, so the other
+// three are at most 2^-23 of a b together, 5.7e-9 in the mean square and of either sign.  (Pieces cut by truncation lost up
+// to 4.7e-7, always towards zero.)
+// Against 64 bits (random normal operands, relative 2-norm) that is closer than fp32 products were: 1.1e-7
+// against 8.1e-7 at K = 1024, 5.4e-8 against 1.46e-7 at K = 33, and without their drift where the operands have one
+// sign: 6.0e-8 against 4.2e-7 at K = 1024.  Where a sum is one product (a diagonal matrix times another) the
+// instruction's own rounding shows: 3.2e-8, at most 1.4e-7, against 2.6e-8 and 6e-8.
+// The matrix rate is what pays for it: 8192 x
 // 1024 x 1024 takes 325 us back to back (515 with v_mfma_f32_32x32x2f32 at 85 % of its peak), 412 GF of bf16
 // products at 1.27 PF; the matrix cores are busy 67 to 68 % of the cycles, at 1.66 to 1.83 GHz by card
 // (rocprofv3; spread thinner, 52 % busy, it clocked 1.95 GHz and took 390 us against 348), probably the power limit.
-// Where one product dominates a sum (operands like exp(6 N(0, 1))) its truncated bits show: up to 1.4e-7.
 //
 // One kernel computes all four real products: each k-step loads the fragments of the three pieces of
 // A_re/A_im and B_re/B_im once from LDS for 24 MFMAs per 32 x 32 tile of the two accumulator sets (the
@@ -31,6 +36,8 @@ namespace tfa {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int GBM = 128, GBN = 128, GBK = 16;
 constexpr int kThreads = 512;
@@ -113,13 +120,14 @@ struct Split {
   unsigned p[3][4];
   template <int C>
   __device__ __forceinline__ void step(const float (&x)[8]) {
-    float r[2] = {x[2 * C], x[2 * C + 1]};
+    floatx2 r = {x[2 * C], x[2 * C + 1]};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      // the two top halves in one register
-      p[q][C] = __builtin_amdgcn_perm(__float_as_uint(r[1]), __float_as_uint(r[0]), 0x07060302u);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) r[h] -= __uint_as_float(__float_as_uint(r[h]) & 0xffff0000u);
+      // both rounded to nearest, in one register
+      const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+      p[q][C] = u;
+      r[0] -= __uint_as_float(u << 16);
+      r[1] -= __uint_as_float(u & 0xffff0000u);
     }
   }
   __device__ __forceinline__ void store(char* dst) const {
@@ -144,10 +152,10 @@ __device__ __forceinline__ int outside(float x) {
   return (!(m < INFINITY) ? 1 : 0) | (m < kTiny && m > 0.0f ? 1 : 0);
 }
 
-// a b + c d over one stage's 16 k, from zero and smallest products first: the instruction truncates its
+// a b + c d over one stage's 16 k, from zero and smallest products first: each instruction rounds its
 // sum, and only the last two products meet a sum of full size here.  (Chained through the whole of K
-// instead, the truncations add up: operands of one sign 2.4e-6 from 64 bits at K = 1024, against
-// 6.0e-7 for fp32 products and 1.1e-7 for these sums added in fp32.)
+// instead, those roundings add up: operands of one sign 2.4e-6 from 64 bits at K = 1024, against
+// 4.2e-7 for fp32 products and 6e-8 for these sums added in fp32.)
 // Step S of 12 is one MFMA of each of two chains: im += A_re B_im + A_im B_re, re += A_re B_re - A_im B_im.
 template <int S>
 __device__ __forceinline__ void product_step(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], const bf16x8 (&nb)[3],
