@@ -304,3 +304,36 @@ def test_gemm_sums_of_one_product(k, value):
     for plane in (got.real, got.imag):
         err = (plane.double() - ref) / ref
         assert err.abs().max() <= 2.0**-22
+
+
+@pytest.mark.parametrize("k", [5, 40])
+@pytest.mark.parametrize("small,large", [(1.99 * 2.0**-120, 2.0**60), (1.2345 * 2.0**-118, 2.0**40), (1.2345 * 2.0**-140, 1.357 * 2.0**100),
+                                         (1.2345 * 2.0**-70, 1.357 * 2.0**-60), (1.99 * 2.0**-103, 1.5)])
+def test_gemm_small_operand_beside_large_ones(k, small, large):
+    # a run of operands whose large value meets a zero: only the small one reaches the sum, at fp32 precision
+    # (test_gemm_sums_of_one_product), and the rest of the tile is as ordinary as ever
+    g = torch.Generator(device="cuda").manual_seed(8)
+    a, b = (torch.randn(*s, generator=g, device="cuda") for s in ((70, k), (k, 90)))
+    a[3, :], b[:, 5] = 0.0, 0.0
+    a[3, 0], a[3, 1] = 1.0, small
+    b[1, 5] = large
+    got = trnfft_amd.complex_matmul(ComplexTensor(a, torch.zeros_like(a)), ComplexTensor(b, torch.zeros_like(b)))
+    want = a[3, 1].double().item() * b[1, 5].double().item()
+    assert abs(got.real[3, 5].double().item() - want) <= 2.0**-22 * want
+    ref = a.double() @ b.double()
+    keep = ref.abs() > 1e-12
+    assert rel_l2(got.real[keep], got.imag[keep], ref[keep], torch.zeros_like(ref[keep])) <= _tol_k(k)
+
+
+@pytest.mark.parametrize("low,high", [(-118, 100), (-126, -60), (60, 126)])
+def test_gemm_scaled_columns(low, high):
+    # A D and D^-1 B for a diagonal D of powers of two: the products, and so the result, are those of A B
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a = tuple(torch.randn(150, 200, generator=g, device="cuda") for _ in range(2))
+    b = tuple(torch.randn(200, 140, generator=g, device="cuda") for _ in range(2))
+    d = 2.0 ** torch.randint(low, high, (200,), generator=g, device="cuda").double()
+    sa = tuple((t.double() * d).float() for t in a)
+    sb = tuple((t.double() / d[:, None]).float() for t in b)
+    got = trnfft_amd.complex_matmul(ComplexTensor(*sa), ComplexTensor(*sb))
+    ref = oracle.complex_matmul(tuple(t.double() for t in sa), tuple(t.double() for t in sb))
+    assert rel_l2(got.real, got.imag, *ref) <= _tol_k(200)

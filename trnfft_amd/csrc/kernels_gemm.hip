@@ -12,7 +12,7 @@
 // to 4.7e-7, always towards zero.)
 // Against 64 bits (random normal operands, relative 2-norm) that is closer than fp32 products were: 1.1e-7
 // against 8.1e-7 at K = 1024, 5.4e-8 against 1.46e-7 at K = 33, and without their drift where the operands have one
-// sign: 6.0e-8 against 4.2e-7 at K = 1024.  Where a sum is one product (a diagonal matrix times another) the
+// sign: 6.0e-8 against 5.9e-7 at K = 1024.  Where a sum is one product (a diagonal matrix times another) the
 // instruction's own rounding shows: 3.2e-8, at most 1.4e-7, against 2.6e-8 and 6e-8.
 // The matrix rate is what pays for it: 8192 x
 // 1024 x 1024 takes 325 us back to back (515 with v_mfma_f32_32x32x2f32 at 85 % of its peak), 412 GF of bf16
@@ -111,10 +111,6 @@ constexpr int kOperand = 2 * kPlane;
 constexpr int kStage = 2 * kOperand;
 static_assert(GBM == GBN, "both operands are staged alike");
 
-// Magnitudes below this leave pieces (2^-24 of the value) in the denormal range, which the bf16
-// matrix instructions flush: operands of 1e-36 lost 5e-5 of the result.
-constexpr float kTiny = 0x1p-100f;
-
 // Eight k of one row, split into their three pieces in four steps of two k.
 struct Split {
   unsigned p[3][4];
@@ -137,25 +133,35 @@ struct Split {
   }
 };
 
-// Whether all of eight values are below kTiny and not all are zero (a run of such values in a row whose
-// other values are larger costs nothing, as the flushed parts are below 2^-24 of those).
-__device__ __forceinline__ int tiny_run(const float (&x)[8]) {
-  float m = 0.0f;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) m = fmaxf(m, fabsf(x[c]));
-  return m < kTiny && m > 0.0f ? 1 : 0;
-}
+// Pieces below 2^-126 lose bits, as bf16 ends at 2^-133 (operands of 1e-36 lost 5e-5 of the result), and so may
+// products of pieces below it.  Such a loss is less than 2^-126 max(1, |a|, |b|) for each of the 12 K real products of a
+// sum, so it shows only in sums that are themselves that small; and where no operand is below kSmall it is at most
+// 2^-30 of its product.  Each thread keeps the least nonzero and the largest magnitude that it splits.  A
+// workgroup that met an operand below kSmall, and has a sum (0 counts) below 2^-96 K max(1, |a|, |b|), takes fp32
+// products; what the others lost is below 12 * 2^-30 of the sum.
+constexpr float kSmall = 0x1p-48f;
+constexpr float kSumLimit = 0x1p-96f;
+struct Range {
+  unsigned lo = ~0u;  // least of 2 bits(|x|) - 1 (zero wraps to the largest)
+  float hi = 0.0f;
+  template <int C>
+  __device__ __forceinline__ void pair(const float (&x)[8]) {
+    const unsigned u = 2 * __float_as_uint(x[2 * C]) - 1, v = 2 * __float_as_uint(x[2 * C + 1]) - 1;
+    lo = min(min(lo, u), v);
+    hi = fmaxf(fmaxf(hi, fabsf(x[2 * C])), fabsf(x[2 * C + 1]));
+  }
+  __device__ __forceinline__ int small() const { return lo < 2 * __float_as_uint(kSmall) - 1 ? 1 : 0; }
+};
 
-// a sum outside the range in which the pieces' products are those of fp32 (zero is inside)
-__device__ __forceinline__ int outside(float x) {
+__device__ __forceinline__ int outside(float x, float limit) {
   const float m = fabsf(x);
-  return (!(m < INFINITY) ? 1 : 0) | (m < kTiny && m > 0.0f ? 1 : 0);
+  return m < INFINITY && m >= limit ? 0 : 1;
 }
 
 // a b + c d over one stage's 16 k, from zero and smallest products first: each instruction rounds its
 // sum, and only the last two products meet a sum of full size here.  (Chained through the whole of K
 // instead, those roundings add up: operands of one sign 2.4e-6 from 64 bits at K = 1024, against
-// 4.2e-7 for fp32 products and 6e-8 for these sums added in fp32.)
+// 5.9e-7 for fp32 products and 6e-8 for these sums added in fp32.)
 // Step S of 12 is one MFMA of each of two chains: im += A_re B_im + A_im B_re, re += A_re B_re - A_im B_im.
 template <int S>
 __device__ __forceinline__ void product_step(const bf16x8 (&a)[2][3], const bf16x8 (&b)[2][3], const bf16x8 (&nb)[3],
@@ -202,7 +208,7 @@ __device__ __forceinline__ void clear(Acc& acc) {
 }
 
 // The tile's sums with fp32 products (v_mfma_f32_32x32x2f32), k from k_begin to K: the pieces of an
-// infinity are not its sum and those of the smallest numbers are flushed, so a workgroup that met either
+// infinity are not its sum and those of the smallest numbers may be flushed, so a workgroup whose sums show either
 // (or an overflow) takes this path over, and its results are those of fp32 arithmetic.
 constexpr int GLD = GBM + 2;  // LDS row pitch in floats (pad 2: transposed stores hit distinct banks)
 static_assert(2 * kStage >= 2 * 2 * GBK * GLD * (int)sizeof(float), "staged in the same LDS");
@@ -243,10 +249,9 @@ __device__ __forceinline__ void tile_f32(float (*As)[GBK][GLD], float (*Bs)[GBK]
   }
 }
 
-// The tile's sums with split products, k from k_begin to K; returns whether this thread met values that
-// need the fp32 path.
+// The tile's sums with split products, k from k_begin to K, and the range of the operands that this thread split.
 template <bool CONJ_B, class OpA, class OpB>
-__device__ __forceinline__ int tile_split(char* smem, int k_begin, const OpA& A, const OpB& B, int w, Acc& acc_re,
+__device__ __forceinline__ Range tile_split(char* smem, int k_begin, const OpA& A, const OpB& B, int w, Acc& acc_re,
                                           Acc& acc_im) {
   const int lane = threadIdx.x & 63, wm = w >> 2, wn = w & 3;
   const int foff = (lane >> 5) * kHalf + (lane & 31) * 16;
@@ -254,14 +259,15 @@ __device__ __forceinline__ int tile_split(char* smem, int k_begin, const OpA& A,
   const int a_dst = A.q.plane * kPlane + A.q.half * kHalf + A.q.row * 16;
   const int b_dst = kOperand + B.q.plane * kPlane + B.q.half * kHalf + B.q.row * 16;
   float xa[8], xb[8];
-  int odd = 0;
+  Range range;
   const auto stage = [&](char* S) {
     Split sa, sb;
     unroll<4>([&](auto c) {
       sa.step<c>(xa);
       sb.step<c>(xb);
+      range.pair<c>(xa);
+      range.pair<c>(xb);
     });
-    odd |= tiny_run(xa) | tiny_run(xb);
     sa.store(S + a_dst);
     sb.store(S + b_dst);
   };
@@ -317,11 +323,10 @@ __device__ __forceinline__ int tile_split(char* smem, int k_begin, const OpA& A,
         if constexpr (s < 4) sa.step<s>(xa);
         else if constexpr (s < 8) sb.step<s - 4>(xb);
         if constexpr (s == 4) sa.store(nxt + a_dst);
-        if constexpr (s == 8) {
-          sb.store(nxt + b_dst);
-          odd |= tiny_run(xa) | tiny_run(xb);
-        }
+        if constexpr (s == 8) sb.store(nxt + b_dst);
         if constexpr (s >= 8) {
+          range.pair<s - 8>(xa);
+          range.pair<s - 8>(xb);
 #pragma unroll
           for (int r = 4 * (s - 8); r < 4 * (s - 7); ++r) {
             acc_im[0][r] += im0[r];
@@ -354,7 +359,7 @@ __device__ __forceinline__ int tile_split(char* smem, int k_begin, const OpA& A,
       acc_re[i] += re;
     }
   }
-  return odd;
+  return range;
 }
 
 // Operands: A_T = op(A) is a transpose (A stored k x m), B_T = op(B) is one (B stored n x k).  Conjugation:
@@ -396,12 +401,26 @@ __global__ __launch_bounds__(kThreads, 2) void cgemm_kernel(
   clear(acc_im);
   const Operand<!A_T> A(A_re, A_im, lda, M, K, row0, t, w);
   const Operand<B_T> B(B_re, B_im, ldb, N, K, col0, t, w);
-  int odd = tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im);
-  // non-finite sums, or sums so small that pieces of the products were flushed
+  const Range range = tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im);
+  // sums below the limit (0 where no operand is small) or not finite need fp32 products
+  float limit = 0.0f;
+  if (__syncthreads_or(range.small())) {
+    float hi = range.hi;
+#pragma unroll
+    for (int d = 32; d > 0; d /= 2) hi = fmaxf(hi, __shfl_xor(hi, d));
+    float* const wave_hi = reinterpret_cast<float*>(smem);
+    if ((t & 63) == 0) wave_hi[w] = hi;
+    __syncthreads();
+    hi = 1.0f;
+#pragma unroll
+    for (int i = 0; i < kThreads / 64; ++i) hi = fmaxf(hi, wave_hi[i]);
+    limit = kSumLimit * (float)(K - k_begin) * hi;
+  }
+  int odd = 0;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) odd |= outside(acc_re[i][r]) | outside(acc_im[i][r]);
+    for (int r = 0; r < 16; ++r) odd |= outside(acc_re[i][r], limit) | outside(acc_im[i][r], limit);
   if (__syncthreads_or(odd)) {
     clear(acc_re);
     clear(acc_im);
