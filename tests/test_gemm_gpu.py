@@ -337,3 +337,38 @@ def test_gemm_scaled_columns(low, high):
     got = trnfft_amd.complex_matmul(ComplexTensor(*sa), ComplexTensor(*sb))
     ref = oracle.complex_matmul(tuple(t.double() for t in sa), tuple(t.double() for t in sb))
     assert rel_l2(got.real, got.imag, *ref) <= _tol_k(200)
+
+
+@pytest.mark.parametrize("k", [16, 17, 40, 512])
+@pytest.mark.parametrize("sa,sb", [(-55, -55), (-50, -65), (-59, -59), (-100, 0), (-105, 0), (-108, -5), (-100, 100), (-16, -100)])
+def test_gemm_sums_around_the_fp32_limit(k, sa, sb):
+    # sums on both sides of the limit below which a workgroup takes fp32 products: 2 k rounded products each way
+    g = torch.Generator(device="cuda").manual_seed(10)
+    a = tuple(torch.randn(140, k, generator=g, device="cuda") * 2.0**sa for _ in range(2))
+    b = tuple(torch.randn(k, 150, generator=g, device="cuda") * 2.0**sb for _ in range(2))
+    got = trnfft_amd.complex_matmul(ComplexTensor(*a), ComplexTensor(*b))
+    ref = oracle.complex_matmul(tuple(t.double() for t in a), tuple(t.double() for t in b))
+    assert rel_l2(got.real, got.imag, *ref) <= 2.0**-24 * math.sqrt(2 * k)
+
+
+@pytest.mark.parametrize("batch,m,k,n", [(1, 1, 1, 1), (3, 129, 16, 127), (700, 5, 7, 3), (300, 16, 16, 16), (2, 130, 17, 260)])
+@pytest.mark.parametrize("a_op,b_op", [(0, 0), (0, 1), (1, 3), (2, 0), (3, 2)])
+def test_gemm_batches_of_one_stage(batch, m, k, n, a_op, b_op):
+    # up to 16 k: one stage of fp32 products, at fp32's own error
+    from trnfft_amd.dispatch import gemm_batched
+
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+
+    def stored(rows, cols, op):
+        shape = (batch, cols, rows) if op in (1, 2) else (batch, rows, cols)
+        return tuple(torch.randn(*shape, generator=g, device="cuda") for _ in range(2))
+
+    def applied(p, op):
+        z = torch.complex(p[0].double().cpu(), p[1].double().cpu())
+        z = z.transpose(1, 2) if op in (1, 2) else z
+        return z.conj().resolve_conj() if op in (2, 3) else z
+
+    a, b = stored(m, k, a_op), stored(k, n, b_op)
+    got = gemm_batched(*a, a_op, *b, b_op, batch, alpha=0.5)
+    ref = 0.5 * (applied(a, a_op) @ applied(b, b_op))
+    assert rel_l2(*got, ref.real, ref.imag) <= 2.0**-24 * math.sqrt(2 * k)

@@ -133,14 +133,14 @@ struct Split {
   }
 };
 
-// Pieces below 2^-126 lose bits, as bf16 ends at 2^-133 (operands of 1e-36 lost 5e-5 of the result), and so may
-// products of pieces below it.  Such a loss is less than 2^-126 max(1, |a|, |b|) for each of the 12 K real products of a
-// sum, so it shows only in sums that are themselves that small; and where no operand is below kSmall it is at most
-// 2^-30 of its product.  Each thread keeps the least nonzero and the largest magnitude that it splits.  A
-// workgroup that met an operand below kSmall, and has a sum (0 counts) below 2^-96 K max(1, |a|, |b|), takes fp32
-// products; what the others lost is below 12 * 2^-30 of the sum.
+// bf16 ends at 2^-133, so operands below 2^-110 lose bits as pieces (operands of 1e-36 lost 5e-5 of the result); the
+// matrix instructions keep denormals.  The loss is at most 2^-133 max(|a|, |b|) for each of the 2 K real products of a
+// sum, or some 2^-149 each where the products are that small, so it shows only in sums that are near that.
+// Each thread keeps the least nonzero and the largest magnitude that it splits.  A
+// workgroup that met an operand below kSmall (without one, products are at least 2^-96), and has a sum (0 counts) below
+// K max(2^-108 |a|, 2^-108 |b|, 2^-118), takes fp32 products; what the others lost is below 2^-24 of the sum.
 constexpr float kSmall = 0x1p-48f;
-constexpr float kSumLimit = 0x1p-96f;
+constexpr float kSumLimit = 0x1p-108f, kSumFloor = 0x1p-118f;
 struct Range {
   unsigned lo = ~0u;  // least of 2 bits(|x|) - 1 (zero wraps to the largest)
   float hi = 0.0f;
@@ -210,15 +210,19 @@ __device__ __forceinline__ void clear(Acc& acc) {
 // The tile's sums with fp32 products (v_mfma_f32_32x32x2f32), k from k_begin to K: the pieces of an
 // infinity are not its sum and those of the smallest numbers may be flushed, so a workgroup whose sums show either
 // (or an overflow) takes this path over, and its results are those of fp32 arithmetic.
+// Two stages in LDS, the next one on its way in registers.  8192 x 1024 x 1024 where every workgroup takes it: 850 us, of which
+// 530 here (with fp32 products alone 512; 880 with one stage in LDS).
 constexpr int GLD = GBM + 2;  // LDS row pitch in floats (pad 2: transposed stores hit distinct banks)
-static_assert(2 * kStage >= 2 * 2 * GBK * GLD * (int)sizeof(float), "staged in the same LDS");
+typedef float F32Stage[2][GBK][GLD];  // [plane][k][row]
+static_assert(2 * kStage >= 4 * (int)sizeof(F32Stage), "staged in the same LDS");
 
+// S: A's and B's stage, and with more than 16 k a second pair
 template <bool CONJ_B, class OpA, class OpB>
-__device__ __forceinline__ void tile_f32(float (*As)[GBK][GLD], float (*Bs)[GBK][GLD], int k_begin, const OpA& A,
-                                         const OpB& B, int w, Acc& acc_re, Acc& acc_im) {
+__device__ __forceinline__ void tile_f32(F32Stage* S, int k_begin, const OpA& A, const OpB& B, int w, Acc& acc_re,
+                                         Acc& acc_im) {
   const int lane = threadIdx.x & 63, wm = w >> 2, wn = w & 3, li = lane & 31, lk = lane >> 5;
-  for (int k0 = k_begin; k0 < A.K; k0 += GBK) {
-    float xa[8], xb[8];
+  float xa[8], xb[8];
+  const auto load = [&](int k0) {
     if (k0 + GBK <= A.K) {
       A.load(k0, xa);
       B.load(k0, xb);
@@ -226,12 +230,23 @@ __device__ __forceinline__ void tile_f32(float (*As)[GBK][GLD], float (*Bs)[GBK]
       A.load_tail(k0, xa);
       B.load_tail(k0, xb);
     }
+  };
+  const auto store = [&](F32Stage* T) {
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-      As[A.q.plane][A.q.half * 8 + c][A.q.row] = xa[c];
-      Bs[B.q.plane][B.q.half * 8 + c][B.q.row] = xb[c];
+      T[0][A.q.plane][A.q.half * 8 + c][A.q.row] = xa[c];
+      T[1][B.q.plane][B.q.half * 8 + c][B.q.row] = xb[c];
     }
-    __syncthreads();
+  };
+  if (k_begin >= A.K) return;
+  load(k_begin);
+  store(S);
+  __syncthreads();
+  int par = 0;
+  for (int k0 = k_begin; k0 < A.K; k0 += GBK, par ^= 2) {
+    const bool more = k0 + GBK < A.K;
+    if (more) load(k0 + GBK);
+    const F32Stage &As = S[par], &Bs = S[par + 1];
 #pragma unroll
     for (int kk = 0; kk < GBK; kk += 2) {
       const float br = Bs[0][kk + lk][wn * 32 + li], b1 = Bs[1][kk + lk][wn * 32 + li];
@@ -245,7 +260,10 @@ __device__ __forceinline__ void tile_f32(float (*As)[GBK][GLD], float (*Bs)[GBK]
         acc_im[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ai, br, acc_im[i], 0, 0, 0);
       }
     }
-    __syncthreads();
+    if (more) {
+      store(S + (par ^ 2));
+      __syncthreads();
+    }
   }
 }
 
@@ -364,15 +382,15 @@ __device__ __forceinline__ Range tile_split(char* smem, int k_begin, const OpA& 
 
 // Operands: A_T = op(A) is a transpose (A stored k x m), B_T = op(B) is one (B stored n x k).  Conjugation:
 // conj(A) op(B) = conj(A conj(op(B))), so CONJ_B is that of exactly one operand, and im_sign is -1 where
-// A is conjugated.
-template <bool A_T, bool B_T, bool CONJ_B>
-__global__ __launch_bounds__(kThreads, 2) void cgemm_kernel(
+// A is conjugated.  SPLIT: products of bf16 pieces; otherwise fp32 products throughout, for at most 16 k.
+template <bool A_T, bool B_T, bool CONJ_B, bool SPLIT>
+__global__ __launch_bounds__(kThreads, SPLIT ? 2 : 4) void cgemm_kernel(
     int M, int N, int K, const float* __restrict__ A_re, const float* __restrict__ A_im, long long lda,
     const float* __restrict__ B_re, const float* __restrict__ B_im, long long ldb, float im_sign,
     const float* __restrict__ bias_re, const float* __restrict__ bias_im, float* __restrict__ C_re,
     float* __restrict__ C_im, long long ldc, float alpha, long long sa, long long sb, long long sc, int k_chunk,
     long long sz) {
-  __shared__ __attribute__((aligned(16))) char smem[2 * kStage];
+  __shared__ __attribute__((aligned(16))) char smem[SPLIT ? 2 * kStage : 2 * sizeof(F32Stage)];
   // batched products: blockIdx.y selects the matrix triple (batch strides in floats; a stride of 0
   // broadcasts one operand over the batch)
   {
@@ -401,31 +419,33 @@ __global__ __launch_bounds__(kThreads, 2) void cgemm_kernel(
   clear(acc_im);
   const Operand<!A_T> A(A_re, A_im, lda, M, K, row0, t, w);
   const Operand<B_T> B(B_re, B_im, ldb, N, K, col0, t, w);
-  const Range range = tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im);
-  // sums below the limit (0 where no operand is small) or not finite need fp32 products
-  float limit = 0.0f;
-  if (__syncthreads_or(range.small())) {
-    float hi = range.hi;
+  if constexpr (SPLIT) {
+    const Range range = tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im);
+    // sums below the limit (0 where no operand is small) or not finite need fp32 products
+    float limit = 0.0f;
+    if (__syncthreads_or(range.small())) {
+      float hi = range.hi;
 #pragma unroll
-    for (int d = 32; d > 0; d /= 2) hi = fmaxf(hi, __shfl_xor(hi, d));
-    float* const wave_hi = reinterpret_cast<float*>(smem);
-    if ((t & 63) == 0) wave_hi[w] = hi;
-    __syncthreads();
-    hi = 1.0f;
+      for (int d = 32; d > 0; d /= 2) hi = fmaxf(hi, __shfl_xor(hi, d));
+      float* const wave_hi = reinterpret_cast<float*>(smem);
+      if ((t & 63) == 0) wave_hi[w] = hi;
+      __syncthreads();
 #pragma unroll
-    for (int i = 0; i < kThreads / 64; ++i) hi = fmaxf(hi, wave_hi[i]);
-    limit = kSumLimit * (float)(K - k_begin) * hi;
-  }
-  int odd = 0;
+      for (int i = 0; i < kThreads / 64; ++i) hi = fmaxf(hi, wave_hi[i]);
+      limit = (float)(K - k_begin) * fmaxf(kSumLimit * hi, kSumFloor);
+    }
+    int odd = 0;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) odd |= outside(acc_re[i][r], limit) | outside(acc_im[i][r], limit);
-  if (__syncthreads_or(odd)) {
-    clear(acc_re);
-    clear(acc_im);
-    auto* S = reinterpret_cast<float (*)[GBK][GLD]>(smem);
-    tile_f32<CONJ_B>(S, S + 2, k_begin, A, B, w, acc_re, acc_im);
+      for (int r = 0; r < 16; ++r) odd |= outside(acc_re[i][r], limit) | outside(acc_im[i][r], limit);
+    if (__syncthreads_or(odd)) {
+      clear(acc_re);
+      clear(acc_im);
+      tile_f32<CONJ_B>(reinterpret_cast<F32Stage*>(smem), k_begin, A, B, w, acc_re, acc_im);
+    }
+  } else {
+    tile_f32<CONJ_B>(reinterpret_cast<F32Stage*>(smem), k_begin, A, B, w, acc_re, acc_im);
   }
   const int li = t & 31, lk = (t >> 5) & 1;
 
@@ -526,8 +546,8 @@ static void launch_cgemm_t(const GemmArgs& a, long long tiles) {
   if (splits > 1) {
     const long long per = a.m * a.n, sz = per * a.batch, plane = sz * splits;
     float* ws = a.workspace;
-    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T, CONJ_B>), dim3((unsigned)tiles, (unsigned)a.batch, splits), dim3(kThreads),
-                       0, a.stream, (int)a.m, (int)a.n, (int)a.k, a.a_re, a.a_im, a.lda, a.b_re, a.b_im, a.ldb,
+    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T, CONJ_B, true>), dim3((unsigned)tiles, (unsigned)a.batch, splits),
+                       dim3(kThreads), 0, a.stream, (int)a.m, (int)a.n, (int)a.k, a.a_re, a.a_im, a.lda, a.b_re, a.b_im, a.ldb,
                        im_sign, nullptr, nullptr, ws, ws + plane, a.n, 1.0f, a.sa, a.sb, per, k_chunk, sz);
     // four columns per thread where every row of C starts 16-byte aligned
     const bool v4 = a.n % 4 == 0 && a.ldc % 4 == 0 && a.sc % 4 == 0 &&
@@ -542,10 +562,13 @@ static void launch_cgemm_t(const GemmArgs& a, long long tiles) {
     else go(cgemm_reduce_kernel<1>, 1);
     return;
   }
+  // At most one stage of k: fp32 products leave room for two workgroups per CU, and no MFMA hides the splitting
+  // (4096 products of 16 x 16 x 16 80 us against 108, 8192 x 16 x 1024 20.7 against 24.3; two stages of split products,
+  // 1000 of 32 x 32 x 32, 39 against 42 for fp32 ones).
+  const auto kern = a.k <= GBK ? cgemm_kernel<A_T, B_T, CONJ_B, false> : cgemm_kernel<A_T, B_T, CONJ_B, true>;
   for (long long b0 = 0; b0 < a.batch; b0 += kMaxGridY) {
     const unsigned nb = (unsigned)std::min(kMaxGridY, a.batch - b0);
-    hipLaunchKernelGGL((cgemm_kernel<A_T, B_T, CONJ_B>), dim3((unsigned)tiles, nb), dim3(kThreads), 0, a.stream, (int)a.m,
-                       (int)a.n, (int)a.k, a.a_re + b0 * a.sa, a.a_im + b0 * a.sa, a.lda, a.b_re + b0 * a.sb,
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, nb), dim3(kThreads), 0, a.stream, (int)a.m, (int)a.n, (int)a.k, a.a_re + b0 * a.sa, a.a_im + b0 * a.sa, a.lda, a.b_re + b0 * a.sb,
                        a.b_im + b0 * a.sb, a.ldb, im_sign, a.bias_re, a.bias_im, a.c_re + b0 * a.sc,
                        a.c_im + b0 * a.sc, a.ldc, a.alpha, a.sa, a.sb, a.sc, k_chunk, 0LL);
   }
