@@ -372,3 +372,29 @@ def test_gemm_batches_of_one_stage(batch, m, k, n, a_op, b_op):
     got = gemm_batched(*a, a_op, *b, b_op, batch, alpha=0.5)
     ref = 0.5 * (applied(a, a_op) @ applied(b, b_op))
     assert rel_l2(*got, ref.real, ref.imag) <= 2.0**-24 * math.sqrt(2 * k)
+
+
+def test_products_and_column_sums_without_memory_for_scratch(monkeypatch):
+    # the scratch of a split product (and of the bias gradient) is an option: without memory for it the call runs unsplit
+    from trnfft_amd import dispatch
+
+    g = torch.Generator(device="cuda").manual_seed(11)
+    m, k, n = 70, 2000, 50
+    a, b = (tuple(torch.randn(*s, generator=g, device="cuda") for _ in range(2)) for s in ((m, k), (k, n)))
+    empty, refused = torch.empty, []
+
+    def no_scratch(*size, **kw):
+        if len(size) == 1 and isinstance(size[0], int):
+            refused.append(size[0])
+            raise torch.OutOfMemoryError("no memory for scratch")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(dispatch.torch, "empty", no_scratch)
+    got = dispatch.gemm_ex(*a, 0, *b, 0)
+    sums = dispatch.column_sums(*b)
+    monkeypatch.undo()
+    assert len(refused) == 2
+    ref = oracle.complex_matmul(tuple(t.double() for t in a), tuple(t.double() for t in b))
+    assert rel_l2(*got, *ref) <= _tol_k(k)
+    # one chain of k / 32 additions between pairwise ones
+    assert rel_l2(*sums, b[0].double().sum(0), b[1].double().sum(0)) <= 2.0**-24 * (4 + math.sqrt(k / 32 + 1))

@@ -169,11 +169,20 @@ def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr() if t is not None else 0)
 
 
+def _scratch(nbytes: int, dev: torch.device) -> torch.Tensor | None:
+    """Device scratch for a faster route, or None where there is no memory for it: the call then takes the
+    route without."""
+    try:
+        return torch.empty(nbytes // 4, dtype=torch.float32, device=dev)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _gemm_workspace(batch: int, m: int, n: int, k: int, dev: torch.device, what: str) -> torch.Tensor | None:
     """Scratch for a product whose k is summed in several ranges at once (None: not split)."""
     nbytes = ctypes.c_size_t()
     _lib.check(_lib.lib().tfa_complex_gemm_workspace_size(batch, m, n, k, ctypes.byref(nbytes)), what)
-    return torch.empty(nbytes.value // 4, dtype=torch.float32, device=dev) if nbytes.value else None
+    return _scratch(nbytes.value, dev) if nbytes.value else None
 
 
 def gemm_ex(a_re, a_im, a_op: int, b_re, b_im, b_op: int, alpha: float = 1.0, bias_re=None, bias_im=None,
@@ -205,7 +214,7 @@ def column_sums(re: torch.Tensor, im: torch.Tensor) -> tuple[torch.Tensor, torch
     if rows >= 64:  # (two chunks of 32 rows at least)
         nbytes = ctypes.c_size_t()
         _lib.check(lib.tfa_column_sums_workspace_size(rows, cols, ctypes.byref(nbytes)), what)
-        ws = re.new_empty(nbytes.value // 4) if nbytes.value else None
+        ws = _scratch(nbytes.value, dev) if nbytes.value else None
     out_re, out_im = re.new_empty(cols), re.new_empty(cols)
     launch(what, dev, lib.tfa_column_sums, rows, cols, addr(re), addr(im), addr(out_re), addr(out_im), addr(ws))
     return out_re, out_im
