@@ -49,6 +49,16 @@ def test_abi_rejects_bad_arguments_without_gpu():
         _lib.check(_lib.TFA_ERR_INVALID, "x")
 
 
+def test_fold_edges_refuses_rows_past_32_bit_indexes():
+    # refused by the arguments alone: the pointer is never followed
+    lib = _lib.lib()
+    big = 2**30
+    for pad, length in [(big - 2, big - 1), (big // 2 + 1, big - 1)]:
+        assert lib.tfa_stft_fold_edges(1, pad, length, 4096, None) == _lib.TFA_ERR_UNSUPPORTED
+    assert lib.tfa_stft_fold_edges(0, 2048, big - 1, 4096, None) == _lib.TFA_OK
+    assert lib.tfa_stft_fold_edges(1, 5, 5, 4096, None) == _lib.TFA_ERR_INVALID
+
+
 def test_create_plan_matches_reference_choice():
     # trnfft/plan.py:34-46
     trnfft_amd.clear_plan_cache()

@@ -426,7 +426,7 @@ __global__ __launch_bounds__(256) void fold_reflect_kernel(float* __restrict__ x
   if (o < 0 || o >= length || (i >= pad && o >= 1 && o <= pad)) return;
   float v = row[pad + o];
   if (o >= 1 && o <= pad) v += row[pad - o];
-  if (o >= length - 1 - pad && o <= length - 2) v += row[pad + 2 * (length - 1) - o];
+  if (o >= length - 1 - pad && o <= length - 2) v += row[pad + (length - 1) + (length - 1 - o)];
   row[pad + o] = v;
 }
 

@@ -1139,7 +1139,8 @@ int tfa_half_rows(int32_t complete, int64_t batch, int64_t n, int64_t half, cons
 int tfa_stft_fold_edges(int64_t batch, int64_t pad, int64_t length, float* grad_padded, tfa_stream stream) {
   if (batch < 0 || pad < 0 || length < 1) return fail(TFA_ERR_INVALID, "bad dimension");
   if (pad >= length) return fail(TFA_ERR_INVALID, "reflect padding needs more samples than pad");
-  if (length > INT32_MAX / 2) return fail(TFA_ERR_UNSUPPORTED, "signal too long");
+  // (the kernel's indexes within a padded row are 32-bit)
+  if (length > INT32_MAX / 2 || length + 2 * pad > INT32_MAX) return fail(TFA_ERR_UNSUPPORTED, "signal too long");
   if (batch == 0 || pad == 0) return TFA_OK;
   if (!grad_padded) return fail(TFA_ERR_INVALID, "null data pointer");
   hipError_t e = tfa::launch_fold_reflect(grad_padded, batch, (int)pad, (int)length, static_cast<hipStream_t>(stream));
