@@ -152,3 +152,21 @@ def test_smooth_stft_nan_stays_in_its_frames():
     bad = torch.isnan(out[1]).nonzero().flatten()
     assert bad.min() >= hit[0] * hop - n // 2 and bad.max() < hit[-1] * hop + n - n // 2
     assert not torch.isnan(out[0]).any()
+
+
+@pytest.mark.parametrize("n", [96, 400, 600])
+@pytest.mark.parametrize("hop", [2**31 + 7, 2**32 + 5, 2**40 + 1])
+def test_smooth_single_frame_at_a_hop_past_int(n, hop):
+    # one frame: the hop's value plays no part, in the inverse and in the gradient (cut to 32 bits it is negative, 5 and 1)
+    win = torch.hann_window(n, device="cuda") + 0.05
+    s = _randn(n, 2, 2, n // 2 + 1, 1)
+    spec = ComplexTensor(s[0], s[1])
+    got, want = (trnfft_amd.istft(spec, n, h, window=win, center=False) for h in (hop, n))
+    zero = torch.zeros_like(got)
+    assert got.shape == (2, n) and rel_l2(got, zero, want, zero) <= 2.0**-22  # (a quotient, or a product with the reciprocal)
+    grads = []
+    for h in (hop, n):
+        x = _randn(n + 1, 2, n + 3).requires_grad_()
+        y = trnfft_amd.stft(x, n, h, window=win, center=False)
+        grads += torch.autograd.grad((y.real, y.imag), (x,), (s[0], s[1]))
+    assert torch.equal(grads[0], grads[1])

@@ -1037,7 +1037,8 @@ int tfa_istft_execute(const tfa_plan* plan, int64_t batch, int64_t n_frames, con
   int64_t out_len = 0;
   int rc = tfa_istft_length(plan, n_frames, length, &out_len);
   if (rc) return rc;
-  const int64_t n_fft = plan->d.n, hop = plan->d.hop;
+  // (a longer hop leaves one frame, whatever its value: kept within int for the kernels)
+  const int64_t n_fft = plan->d.n, hop = std::min<int64_t>(plan->d.hop, INT32_MAX / 2);
   const bool two_sided = !(plan->d.flags & TFA_STFT_ONESIDED);
   const int64_t expected = n_fft + (n_frames - 1) * hop;
   if (expected > INT32_MAX / 2 || n_frames > INT32_MAX / 2 || out_len > INT32_MAX / 2 ||
@@ -1078,7 +1079,7 @@ int tfa_stft_backward_execute(const tfa_plan* plan, int64_t batch, int64_t n_fra
     return fail(TFA_ERR_INVALID, "the STFT backward runs on the forward STFT plan");
   if (!(plan->d.flags & TFA_STFT_ONESIDED)) return fail(TFA_ERR_UNSUPPORTED, "the fused STFT backward takes onesided spectra");
   if (batch < 0) return fail(TFA_ERR_INVALID, "negative batch");
-  const int64_t n_fft = plan->d.n, hop = plan->d.hop;
+  const int64_t n_fft = plan->d.n, hop = std::min<int64_t>(plan->d.hop, INT32_MAX / 2);  // (as in tfa_istft_execute)
   const bool pow2 = is_pow2(n_fft);
   // the adjoint kernels tile like the inverse ones: a halo of floor((n-1)/hop) recomputed frames
   const int64_t halo = (n_fft - 1) / hop;
