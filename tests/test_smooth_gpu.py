@@ -154,6 +154,18 @@ def test_smooth_stft_nan_stays_in_its_frames():
     assert not torch.isnan(out[0]).any()
 
 
+@pytest.mark.parametrize("n", LENGTHS)
+def test_smooth_rows_of_tones(n):
+    # the direct transform of tones, on and between bins, is the exact one too (the reference's fp32 chirp errs most there)
+    f = torch.cat([torch.arange(0, n, max(1, n // 20)).double(), torch.rand(20, generator=torch.Generator().manual_seed(n)).double() * n])
+    z = torch.exp(2j * torch.pi * f[:, None] * torch.arange(n) / n)
+    x = ComplexTensor(z.real.float().cuda(), z.imag.float().cuda())
+    ref = torch.fft.fft(_z(x.real, x.imag))
+    y = trnfft_amd.fft(x)
+    for i in range(len(f)):
+        assert rel_l2(y.real[i], y.imag[i], ref.real[i], ref.imag[i]) <= tol_pow2(n)
+
+
 @pytest.mark.parametrize("n", [96, 400, 600])
 @pytest.mark.parametrize("hop", [2**31 + 7, 2**32 + 5, 2**40 + 1])
 def test_smooth_single_frame_at_a_hop_past_int(n, hop):

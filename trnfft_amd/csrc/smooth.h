@@ -4,10 +4,12 @@
 //
 // The reference runs Bluestein's chain at these lengths with chirp angles pi k^2 / n rounded to fp32, which
 // is what its results differ by from the exact transform: about 1.15e-7 n, growing with n.  The direct
-// transform has no such error (1e-7), so it differs from the reference's result by the reference's own: on
-// random rows 0.46 of the parity bound 1e-5 log2 n at n = 400, 0.67 at 500 and 0.76 at 640 (measured over
-// all these lengths), past the bound from 875 on.  Hence the limit of 640; longer lengths, and lengths with
-// other factors, follow the reference's chain.
+// transform has no such error (1e-7, and is held to 1e-6 log2 n of float64), so it differs from the reference's result by
+// the reference's own.  In parts of the parity bound 1e-5 log2 n that is, on random rows, 0.48 at n = 400, 0.67 at 500, 0.75
+// at 640, 0.73 to 0.83 from 648 to 720 and past it from 875 on; a tone meets the chirp's worst angles: at most 1.0
+// below 256, up to 2.4 at 600 and 640 (2.0 where it is Hann-windowed).  Longer lengths are further off, and the kernels were
+// measured and tested up to the 640 points of a camera's row: from there on, and at lengths with other factors, rows follow
+// the reference's chain.
 #pragma once
 #include <initializer_list>
 #include <type_traits>
