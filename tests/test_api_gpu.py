@@ -121,7 +121,7 @@ def test_stft_vs_oracle(n_fft, hop, center, normalized, onesided):
 
 
 @pytest.mark.parametrize("n_fft,hop,pad_mode,center,onesided,normalized,shape", [
-    (400, 160, "reflect", True, True, False, (2, 16000)),      # 25 ms @ 16 kHz: a Bluestein transform per frame
+    (400, 160, "reflect", True, True, False, (2, 16000)),      # 25 ms @ 16 kHz: a direct transform per frame
     (400, 100, "constant", True, True, True, (3, 5000)),
     (12, 3, "replicate", True, True, False, (2, 301)),         # the fused kernel's shortest convolution (32)
     (12, 5, "circular", True, False, False, (1, 200)),         # (1, L): the reference squeezes the batch axis
@@ -156,15 +156,22 @@ def test_stft_any_n_fft_and_pad_mode_vs_oracle(n_fft, hop, pad_mode, center, one
     (30, 12, True, True, False, (2, 1500)),      # m = 64
     (33, 11, True, False, False, (1, 999)),      # m = 96, two-sided
     (50, 20, True, True, False, (2, 2000)),      # m = 96
-    (80, 30, False, True, False, (2, 2500)),     # m = 128
-    (100, 40, True, True, False, (4, 3001)),     # m = 192
+    (80, 30, False, True, False, (2, 2500)),     # a direct transform, as the other lengths so marked
+    (70, 30, False, True, False, (2, 2500)),     # m = 128
+    (100, 40, True, True, False, (4, 3001)),     # direct
+    (118, 40, True, True, False, (4, 3001)),     # m = 192
     (150, 60, True, True, True, (2, 4000)),      # m = 256
-    (200, 64, True, True, False, (2, 8000)),     # m = 384
+    (200, 64, True, True, False, (2, 8000)),     # direct
+    (202, 64, True, True, False, (2, 8000)),     # m = 384
     (257, 128, True, True, False, (2, 5000)),    # m = 512
-    (300, 450, False, True, False, (2, 9000)),   # m = 512, hop > n_fft
-    (400, 160, True, True, False, (3, 16000)),   # m = 768
-    (400, 160, True, True, False, (2, 201)),     # every frame reaches into the reflect padding
-    (640, 160, False, True, True, (2, 9000)),    # m = 1024
+    (300, 450, False, True, False, (2, 9000)),   # direct, hop > n_fft
+    (302, 450, False, True, False, (2, 9000)),   # m = 512, hop > n_fft
+    (400, 160, True, True, False, (3, 16000)),   # direct
+    (400, 160, True, True, False, (2, 201)),     # direct, every frame reaches into the reflect padding
+    (441, 160, True, True, False, (3, 16000)),   # m = 768
+    (441, 160, True, True, False, (2, 221)),     # every frame reaches into the reflect padding
+    (640, 160, False, True, True, (2, 9000)),    # direct
+    (642, 160, False, True, True, (2, 9000)),    # m = 1024
     (1000, 250, True, True, False, (2, 7000)),   # m = 1536
     (1000, 250, True, False, False, (2, 7000)),  # m = 2048, two-sided
     (1025, 300, True, True, False, (2, 9000)),   # m = 2048
@@ -174,7 +181,8 @@ def test_stft_any_n_fft_and_pad_mode_vs_oracle(n_fft, hop, pad_mode, center, one
 ])
 def test_stft_fused_bluestein_frames_vs_oracle(n_fft, hop, center, onesided, normalized, shape):
     # n_fft that is not a power of two, without autograd: one fused kernel with a Bluestein
-    # transform per frame (the reference's chain, trnfft/api.py:339-349 -> fft_core.py:1285-1376)
+    # transform per frame (the reference's chain, trnfft/api.py:339-349 -> fft_core.py:1285-1376),
+    # or a direct one where n_fft is a multiple of 4 from 36 to 640 without a prime factor above 7
     g = torch.Generator().manual_seed(n_fft * 7 + hop)
     x = torch.randn(*shape, generator=g)
     got = trnfft_amd.stft(x.cuda(), n_fft=n_fft, hop_length=hop, center=center, normalized=normalized,
@@ -184,11 +192,12 @@ def test_stft_fused_bluestein_frames_vs_oracle(n_fft, hop, center, onesided, nor
     assert rel_l2(got.real, got.imag, *ref) <= tol_bluestein(n_fft)
 
 
-@pytest.mark.parametrize("n_fft,hop,pad_mode", [(400, 160, "reflect"), (1000, 256, "constant"), (99, 33, "circular")])
+@pytest.mark.parametrize("n_fft,hop,pad_mode", [(441, 160, "reflect"), (1000, 256, "constant"), (99, 33, "circular"),
+                                                (400, 160, "reflect")])
 def test_stft_fused_bluestein_matches_composed_path(n_fft, hop, pad_mode):
     # the reference's composition on the device (pad, frame gather, window, Bluestein rows of
-    # rfft, transpose) against the fused kernel: both run the reference's chain, so they agree
-    # to fp32 rounding
+    # rfft, transpose) against the fused kernel: both run the reference's chain (both the direct
+    # transform at 400), so they agree to fp32 rounding
     g = torch.Generator().manual_seed(13)
     x = torch.randn(3, 12000, generator=g).cuda()
     fused = trnfft_amd.stft(x, n_fft=n_fft, hop_length=hop, pad_mode=pad_mode)

@@ -156,11 +156,13 @@ def test_strided_axis_gradient():
     assert rel_l2(a_r.grad, a_i.grad, r_r.grad, r_i.grad) <= TOL
 
 
-def test_strided_non_pow2_axis_gradient():
-    # a Bluestein length down a strided axis: forward and adjoint both on the strided kernel
+@pytest.mark.parametrize("n", [100, 102])
+def test_strided_non_pow2_axis_gradient(n):
+    # a length down a strided axis that is no power of two (100: direct, 102: Bluestein): forward and adjoint
+    # both on the strided kernel
     g = torch.Generator().manual_seed(14)
-    xr, xi = torch.randn(3, 100, 24, generator=g), torch.randn(3, 100, 24, generator=g)
-    cr, ci = _cotangent((3, 100, 24), 15)
+    xr, xi = torch.randn(3, n, 24, generator=g), torch.randn(3, n, 24, generator=g)
+    cr, ci = _cotangent((3, n, 24), 15)
     a_r, a_i = _leaf(xr), _leaf(xi)
     y = trnfft_amd.fftn(ComplexTensor(a_r, a_i), dim=(1,))
     (y.real * cr.float().cuda() + y.imag * ci.float().cuda()).sum().backward()
@@ -256,20 +258,27 @@ def test_stft_gradient_fused_backward(n_fft, hop, center, normalized, shape, mon
 
 
 @pytest.mark.parametrize("n_fft,hop,center,normalized,shape", [
-    (400, 160, True, False, (2, 4000)),       # convolution length 768
+    (441, 160, True, False, (2, 4000)),       # convolution length 768
+    (441, 110, False, True, (2, 3, 3000)),
+    (400, 160, True, False, (2, 4000)),       # direct transforms
     (400, 100, False, True, (2, 3, 3000)),
     (12, 4, True, False, (2, 301)),           # 32
     (30, 10, True, False, (2, 500)),          # 64
-    (100, 40, True, False, (2, 2000)),        # 192
+    (100, 40, True, False, (2, 2000)),        # direct
+    (99, 40, True, False, (2, 2000)),         # 192
+    (130, 40, True, False, (2, 2000)),        # 256
+    (202, 80, True, False, (2, 3000)),        # 384
     (257, 128, True, False, (2, 3000)),       # 512
-    (600, 200, True, False, (1, 5000)),       # 1024
+    (600, 200, True, False, (1, 5000)),       # direct
+    (602, 200, True, False, (1, 5000)),       # 1024
     (1000, 300, True, True, (1, 6000)),       # 1536
     (2000, 1000, True, False, (1, 9000)),     # 3072
-    (400, 500, True, False, (2, 2000)),       # hop > n_fft
+    (400, 500, True, False, (2, 2000)),       # direct, hop > n_fft
+    (441, 500, True, False, (2, 2000)),       # hop > n_fft
 ])
 def test_stft_gradient_fused_backward_non_pow2(n_fft, hop, center, normalized, shape, monkeypatch):
-    # n_fft that is not a power of two, window without gradient: the adjoint Bluestein chain per
-    # frame in one kernel, against autograd through the oracle's restatement of the reference's
+    # n_fft that is not a power of two, window without gradient: the adjoint Bluestein chain (or direct
+    # transform) per frame in one kernel, against autograd through the oracle's restatement of the reference's
     # pytorch path (the reference's operator carries its fp32 chirp)
     from trnfft_amd import fft_core
 
@@ -349,7 +358,7 @@ def test_stft_gradient_composed_pow2(n_fft, hop, pad_mode):
 
 
 def test_stft_gradient_composed_bluestein():
-    # n_fft = 400 (Bluestein frames): against autograd through the oracle's restatement of the
+    # n_fft = 400 (direct transforms; the oracle's Bluestein frames): against autograd through the oracle's restatement of the
     # reference's own pytorch path in fp32 (its fp32 chirp differs from the exact DFT)
     g = torch.Generator().manual_seed(17)
     x = torch.randn(2, 4000, generator=g)

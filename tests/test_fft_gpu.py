@@ -194,7 +194,9 @@ def test_bluestein_vs_reference_golden(direction):
                                      # workgroup): full tiles plus a ragged one, every padded length
                                      # 4..256 and real input below
                                      (2, 600), (5, 1000), (7, 257), (12, 300), (31, 513), (33, 129),
-                                     (60, 200), (100, 130), (127, 65), (129, 3)])
+                                     (60, 200), (100, 130), (127, 65), (129, 3),
+                                     # (60, 100 and their like, 36 to 640, transform directly:) lengths beside them
+                                     (62, 200), (102, 130), (255, 70), (382, 40), (510, 20)])
 @pytest.mark.parametrize("inverse", [False, True])
 def test_bluestein_vs_oracle(n, batch, inverse):
     re, im = seeded_complex(batch, n, seed=n)
@@ -203,7 +205,7 @@ def test_bluestein_vs_oracle(n, batch, inverse):
     assert rel_l2(*got, *ref) <= tol_bluestein(n), (n, inverse)
 
 
-@pytest.mark.parametrize("n", [3, 12, 100])
+@pytest.mark.parametrize("n", [3, 12, 31, 100, 102])
 def test_bluestein_short_rows_real_input(n):
     re, _ = seeded_complex(301, n, seed=n + 1)
     X = trnfft_amd.fft(re.cuda())
@@ -211,7 +213,8 @@ def test_bluestein_short_rows_real_input(n):
     assert rel_l2(X.real, X.imag, *ref) <= tol_bluestein(n)
 
 
-@pytest.mark.parametrize("n,batch,real_in", [(257, 40, False), (300, 64, True), (384, 33, False), (513, 20, False),
+@pytest.mark.parametrize("n,batch,real_in", [(257, 40, False), (302, 64, True), (383, 33, False), (513, 20, False),
+                                              (300, 64, True), (384, 33, False),  # (direct transforms)
                                               (700, 17, True), (768, 9, False), (1025, 12, False), (1300, 7, True),
                                               (1536, 5, False), (1537, 3, False), (4200, 9, False)])
 def test_bluestein_mixed_radix_lengths_vs_oracle(n, batch, real_in):
@@ -274,6 +277,18 @@ def test_bluestein_two_level_lengths_vs_oracle(n, batch, inverse):
     X = trnfft_amd.ifft(re.cuda()) if inverse else trnfft_amd.fft(re.cuda())
     ref = oracle.fft_core(re, torch.zeros_like(re), inverse)
     assert rel_l2(X.real, X.imag, *ref) <= tol_bluestein(n), (n, inverse, "real input")
+
+
+@pytest.mark.parametrize("n", [3, 7, 13, 31, 62, 127, 254, 510, 1021, 2047])
+@pytest.mark.parametrize("width", [1, 37])
+def test_bluestein_strided_axis_every_length_vs_oracle(n, width):
+    # the longest axes but one or two of each convolution length 8 to 4096 that no direct transform takes
+    g = torch.Generator().manual_seed(n)
+    re, im = torch.randn(3, n, width, generator=g), torch.randn(3, n, width, generator=g)
+    for inverse in (False, True):
+        got = (trnfft_amd.ifftn if inverse else trnfft_amd.fftn)(ComplexTensor(re.cuda(), im.cuda()), dim=(1,))
+        ref = oracle.fft_core(re.transpose(1, 2).contiguous(), im.transpose(1, 2).contiguous(), inverse)
+        assert rel_l2(got.real.transpose(1, 2), got.imag.transpose(1, 2), *ref) <= tol_bluestein(n), inverse
 
 
 @pytest.mark.parametrize("n", [1027, 4099])

@@ -199,21 +199,29 @@ def test_istft_small_hop_falls_back_to_composition():
 
 
 BLUE_CASES = [
-    # n_fft, hop, frames, center, normalized, length; m = the inverse chain's length (>= 2 n_fft - 1)
-    (400, 160, 101, True, False, None),     # m 1024
-    (400, 100, 60, True, True, None),
-    (320, 160, 50, True, False, 9000),      # m 768; longer length: zero fill
+    # n_fft, hop, frames, center, normalized, length; m = the inverse chain's length (>= 2 n_fft - 1), or
+    # direct: multiples of 4 from 36 to 640 without a prime factor above 7
+    (400, 160, 101, True, False, None),     # direct
+    (400, 100, 60, True, True, None),       # direct
+    (441, 160, 101, True, False, None),     # m 1024
+    (441, 110, 60, True, True, None),
+    (320, 160, 50, True, False, 9000),      # direct; longer length: zero fill
+    (350, 160, 50, True, False, 9000),      # m 768; longer length: zero fill
     (9, 2, 40, True, False, None),          # m 32
     (12, 3, 80, True, False, None),
     (30, 7, 70, False, False, None),        # m 64
-    (40, 10, 50, True, False, None),        # m 96
+    (40, 10, 50, True, False, None),        # direct
+    (45, 11, 50, True, False, None),        # m 96
     (50, 60, 20, False, False, None),       # m 128; hop > n_fft
     (90, 30, 40, True, False, None),        # m 192
     (99, 33, 30, True, False, None),        # m 256; odd n_fft
-    (100, 25, 40, True, False, 900),        # shorter length: truncation
+    (100, 25, 40, True, False, 900),        # direct; shorter length: truncation
+    (101, 25, 40, True, False, 900),        # m 256; shorter length: truncation
     (150, 50, 30, True, True, None),        # m 384
-    (200, 80, 30, True, False, None),       # m 512
-    (600, 150, 20, True, False, None),      # m 1536
+    (200, 80, 30, True, False, None),       # direct
+    (230, 80, 30, True, False, None),       # m 512
+    (600, 150, 20, True, False, None),      # direct
+    (602, 150, 20, True, False, None),      # m 1536
     (1000, 250, 12, False, True, None),     # m 2048
     (1500, 750, 9, True, False, None),      # m 3072
     (2047, 1024, 6, True, False, None),     # m 4096
@@ -222,7 +230,7 @@ BLUE_CASES = [
 
 @pytest.mark.parametrize("n_fft,hop,frames,center,normalized,length", BLUE_CASES)
 def test_istft_non_pow2_matches_reference(n_fft, hop, frames, center, normalized, length):
-    # one inverse Bluestein chain per frame (the reference's fp32 chirp), fused with the
+    # one inverse Bluestein chain per frame (the reference's fp32 chirp) or direct transform, fused with the
     # completion, window, overlap-add and envelope
     from conftest import tol_bluestein
 
@@ -235,7 +243,7 @@ def test_istft_non_pow2_matches_reference(n_fft, hop, frames, center, normalized
     assert trnfft_amd.api._istft_fused(x, n_fft, hop, n_fft, None, center, normalized, True, length) is not None
 
 
-@pytest.mark.parametrize("n_fft,hop,frames", [(400, 10, 120), (2047, 512, 8)])
+@pytest.mark.parametrize("n_fft,hop,frames", [(400, 10, 120), (441, 11, 120), (2047, 512, 8)])
 def test_istft_non_pow2_small_hop_composes(n_fft, hop, frames):
     # a halo of more than half the fused tile: the composed path (frame inverse transforms +
     # overlap-add)
@@ -250,7 +258,7 @@ def test_istft_non_pow2_small_hop_composes(n_fft, hop, frames):
 
 
 def test_stft_istft_roundtrip_non_pow2():
-    # C2's signals at n_fft 400 / hop 160 through both fused per-frame Bluestein kernels
+    # 16 kHz signals at n_fft 400 / hop 160 through both fused direct-transform kernels
     from bench import make_stft_input
 
     x = make_stft_input(8, 160000).cuda()

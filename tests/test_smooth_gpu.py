@@ -88,7 +88,8 @@ def _stft64(x, n, hop, win):
 
 @pytest.mark.parametrize("n", LENGTHS)
 def test_smooth_stft_inverse_and_gradient(n):
-    # 70 frames: a whole tile and a partial one; the signal short enough that both edges reflect
+    # 70 frames of two signals: the forward kernel's quarter tiles (the full ones below), a whole and a partial tile of
+    # the inverse and the gradient; the signal short enough that both edges reflect
     hop = (2 * n) // 5
     x = _randn(n, 2, 69 * hop + 3)
     win = torch.hann_window(n, device="cuda") + 0.05
@@ -152,6 +153,69 @@ def test_smooth_stft_nan_stays_in_its_frames():
     bad = torch.isnan(out[1]).nonzero().flatten()
     assert bad.min() >= hit[0] * hop - n // 2 and bad.max() < hit[-1] * hop + n - n // 2
     assert not torch.isnan(out[0]).any()
+
+
+def _frames_per_tile(n):
+    return 64 if n <= 128 else 32 if n <= 448 else 16
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_smooth_stft_full_tiles(n):
+    # calls of 256 tiles or more take the full tile: one whole and one of five frames per signal, 260 in all; a hop whose
+    # span the areas hold, and one whose frames are read one by one
+    fr = _frames_per_tile(n)
+    win = torch.hann_window(n, device="cuda") + 0.05
+    for hop in ((2 * n) // 5 + 1, 2 * n + 3):
+        x = _randn(n + hop, 130, (fr + 4) * hop + 3)
+        ref = _stft64(x.double(), n, hop, win.double())
+        assert ref.shape[-1] == fr + 5
+        y = trnfft_amd.stft(x, n, hop, window=win)
+        assert rel_l2(y.real, y.imag, ref.real, ref.imag) <= tol_pow2(n)
+        if n not in (36, 60, 120, 140, 196, 384, 392, 400, 432, 448, 480, 640):
+            continue
+        fm = trnfft_amd.stft(x, n, hop, window=win, frames_major=True)
+        assert torch.equal(fm.real, y.real) and torch.equal(fm.imag, y.imag)
+        for frames_major in (False, True):
+            two = trnfft_amd.stft(x, n, hop, window=win, onesided=False, frames_major=frames_major)
+            h = n // 2 + 1
+            assert torch.equal(two.real[:, :h], y.real) and torch.equal(two.imag[:, :h], y.imag)
+            assert torch.equal(two.real[:, h:], y.real[:, 1 : h - 1].flip(1))
+            assert torch.equal(two.imag[:, h:], -y.imag[:, 1 : h - 1].flip(1))
+
+
+@pytest.mark.parametrize("frames_major", [False, True])
+@pytest.mark.parametrize("n,hop", [(36, 4), (60, 7), (96, 3), (96, 11), (120, 15), (120, 23), (140, 17), (200, 25), (200, 39), (400, 50),
+                                   (400, 99), (448, 56), (480, 60), (480, 96), (600, 120), (640, 130), (640, 150)])
+def test_smooth_inverse_and_gradient_of_many_overlaps(n, hop, frames_major):
+    # five to 32 frames over each sample (halos of 4 and more): the overlap-add's general form, over several tiles
+    halo = (n - 1) // hop
+    assert halo >= 4
+    frames = 3 * _frames_per_tile(n) + 7
+    win = torch.hann_window(n, device="cuda") + 0.05
+    w64 = win.double()
+    shape = (2, 2, frames, n // 2 + 1) if frames_major else (2, 2, n // 2 + 1, frames)
+    g = _randn(n + hop, *shape)
+    g = g.transpose(-2, -1) if frames_major else g
+    g64 = torch.complex(g[0].double(), g[1].double())
+    spec = ComplexTensor._wrap(g[0], g[1])
+    got = trnfft_amd.istft(spec, n, hop, window=win)
+    assert trnfft_amd.api._istft_fused(spec, n, hop, n, win, True, False, True, None) is not None
+    y = torch.fft.irfft(g64.transpose(-2, -1), n=n, dim=-1) * w64
+    total = n + (frames - 1) * hop
+    pos = (torch.arange(frames, device="cuda")[:, None] * hop + torch.arange(n, device="cuda")).reshape(-1)
+    out = torch.zeros(2, total, dtype=torch.float64, device="cuda").index_add_(1, pos, y.reshape(2, -1))
+    env = torch.zeros(total, dtype=torch.float64, device="cuda").index_add_(0, pos, (w64 * w64).repeat(frames))
+    want = (out / env)[:, n // 2 : total - n // 2]
+    assert rel_l2(got, torch.zeros_like(got), want, torch.zeros_like(want)) <= 2 * tol_pow2(n)
+    # the gradient (the composed adjoint where the kernel's tile has no room for the halo)
+    x = _randn(n, 2, (frames - 1) * hop).requires_grad_()
+    x64 = x.detach().double().requires_grad_()
+    z = trnfft_amd.stft(x, n, hop, window=win, frames_major=frames_major)
+    ref = _stft64(x64, n, hop, w64)
+    assert z.real.shape == ref.shape == g[0].shape
+    (got,) = torch.autograd.grad((z.real, z.imag), (x,), (g[0], g[1]))
+    (want,) = torch.autograd.grad((ref.real, ref.imag), (x64,), (g64.real, g64.imag))
+    assert rel_l2(got, torch.zeros_like(got), want, torch.zeros_like(want)) <= 2 * tol_pow2(n)
 
 
 @pytest.mark.parametrize("n", LENGTHS)
