@@ -9,8 +9,8 @@ reference checkout:
     python tests/golden/make_bluestein_vectors.py
 
 Output: tests/golden/bluestein_vectors.npz with, per case, the seeded inputs and the
-reference's fft and ifft outputs.  The GPU box never runs this script (the reference is not
-there); tests only read the .npz.
+reference's fft and ifft outputs.  Only a machine that holds the reference can run this script;
+tests only read the .npz.
 """
 
 from __future__ import annotations
@@ -25,7 +25,7 @@ REF = "/root/reference"
 OUT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "bluestein_vectors.npz")
 
 # (n, batch): the reference tests' arbitrary sizes (tests/conftest.py:21-23) plus the two
-# BASELINE Bluestein lengths at small batch.
+# benchmark's Bluestein lengths at small batch.
 CASES = [(7, 3), (11, 2), (100, 3), (127, 2), (997, 2), (1000, 4), (4099, 2)]
 
 

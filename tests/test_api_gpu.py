@@ -94,7 +94,7 @@ def test_fftn_ifftn():
 
 
 def test_fft2_config4a_one_image_and_parseval():
-    # BASELINE config 4a at full shape (32 x 2048 x 2048, U[0,1)): oracle on one image, Parseval on all
+    # the benchmark's images at full shape (32 x 2048 x 2048, U[0,1)): oracle on one image, Parseval on all
     g = torch.Generator().manual_seed(42)
     x = torch.rand(32, 2048, 2048, generator=g)
     got = trnfft_amd.fft2(x.cuda())
@@ -235,7 +235,7 @@ def test_stft_result_layout_is_the_references(n_fft, hop):
 
 
 @pytest.mark.parametrize("n_fft,hop,shape,center", [
-    (512, 256, (64, 160000), True),    # 626 frames, 4 ranges per signal, 256 workgroups
+    (512, 256, (64, 160000), True),    # the benchmark's STFT: 626 frames, 4 ranges per signal, 256 workgroups
     (512, 256, (1, 40192), True),      # one signal (158 frames): ranges of one sub-tile and a half
     (512, 128, (3, 9100), True),       # 72 frames: two ranges of 36
     (512, 300, (5, 50100), False),     # no padding; hop not a divisor of n_fft (166 frames)
@@ -309,7 +309,7 @@ def test_stft_no_whole_frame_returns_empty_like_the_reference():
 
 
 def test_stft_config2_full_size():
-    # 64 x 160000 samples, 3 sinusoids + N(0, 0.1) noise, n_fft 512, hop 256
+    # the benchmark's STFT: 64 x 160000 samples, 3 sinusoids + N(0, 0.1) noise, n_fft 512, hop 256
     from bench import make_stft_input
 
     x = make_stft_input(64, 160000, seed=42)

@@ -115,7 +115,7 @@ def test_pow2_fourstep_real_input(n):
 
 
 def test_config1_batched_1024_roundtrip():
-    # 4096 x 1024, forward then inverse, each against the oracle
+    # the benchmark's batch: 4096 x 1024, forward then inverse, each against the oracle
     re, im = seeded_complex(4096, 1024)
     x = ComplexTensor(re.cuda(), im.cuda())
     X = trnfft_amd.fft(x)
@@ -128,7 +128,7 @@ def test_config1_batched_1024_roundtrip():
 
 
 def test_config4b_large_n_properties():
-    # BASELINE config 4b at full size (16 x 2^20): oracle on one row, round trip + Parseval on all
+    # the benchmark's long rows at full size (16 x 2^20): oracle on one row, round trip + Parseval on all
     n = 1 << 20
     re, im = seeded_complex(16, n)
     x = ComplexTensor(re.cuda(), im.cuda())

@@ -130,7 +130,7 @@ def test_dft_gemm_vs_oracle(n, inverse):
 
 
 def test_config5b_full_size_both_formulations():
-    # BASELINE config 5b at full size (65536 x 256, forward): the DFT-as-GEMM on the matrix cores
+    # the benchmark's DFT as a product at full size (65536 x 256, forward): the DFT-as-GEMM on the matrix cores
     # and the Stockham kernel, each against the oracle on all rows
     from trnfft_amd import fft_core as fc
 

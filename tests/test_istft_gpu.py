@@ -55,7 +55,7 @@ CASES = [
 # leading dims
 RANGE_CASES = [
     # lead, n_fft, hop, frames, center, normalized, length
-    ((64,), 512, 256, 626, True, False, None),    # BASELINE config 2's inverse
+    ((64,), 512, 256, 626, True, False, None),    # the benchmark's STFT, inverted
     ((1,), 512, 256, 2000, True, False, None),    # one signal
     ((2,), 512, 256, 627, True, False, None),     # odd frame count
     ((300,), 512, 256, 70, True, False, None),    # more signals than CUs
@@ -179,7 +179,7 @@ def test_istft_leading_dims_and_win_length():
 
 
 def test_stft_istft_roundtrip_full_size():
-    # BASELINE config 2 shape: 64 waveforms x 160000 samples, n_fft 512, hop 256
+    # the benchmark's shape: 64 waveforms x 160000 samples, n_fft 512, hop 256
     from bench import make_stft_input
 
     x = make_stft_input(64, 160000).cuda()

@@ -17,7 +17,7 @@
 //      and the output scale, first n entries stored.
 // The spectrum is never brought back to natural order: the filter multiply happens in the
 // transposed domain, so the chain is three passes (the intermediate, batch*m*8 bytes, stays in
-// the Infinity Cache at the BASELINE sizes) instead of two full four-step transforms.
+// the Infinity Cache at the benchmark's sizes) instead of two full four-step transforms.
 #include "kernels.h"
 
 namespace tfa {

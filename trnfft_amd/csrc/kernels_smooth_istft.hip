@@ -14,7 +14,9 @@
 
 namespace tfa {
 
-// Frames per workgroup: above the longest halo that the plan accepts (32 frames up to n_fft 128, else 16)
+// Frames per workgroup: above the longest halo that the plan accepts (32 frames up to n_fft 128, else 16), which asks for 64 up
+// to 128; 20 is what LDS holds at n_fft 640.  64 signals, 160000 samples, hop 2n/5: n_fft 140 44.6 us with 64 frames and 37.9 with 32,
+// 168 40.2 and 38.5; with 32 and with 20, 420 51.8 and 53.0, 432 63.8 and 48.4, 448 50.0 and 46.5.
 template <int N>
 constexpr int smooth_istft_frames() {
   return N <= 128 ? 64 : N <= 448 ? 32 : 20;

@@ -126,7 +126,10 @@ struct SmoothGroup {
 };
 
 constexpr int kSmoothLds3 = 53760;  // LDS that lets three workgroups share a CU (160 KB in units of 1280 bytes)
-// Whether XF areas of N points, and `more` bytes, take three workgroups per CU only without padding
+// Padded, unless XF areas of N points, and `more` bytes, let three workgroups share the CU only without padding.  That takes
+// 64 x 160000 samples, STFT and inverse, from 43.4 to 37.2 us and 52.9 to 44.2 at n_fft 392, from 42.5 to 40.2 and 56.9 to 54.8 at
+// 400.  A pitch that is a multiple of 8 keeps the padding, as its lanes would share banks: at 384 (N2 = 16) the inverse
+// takes 45.2 us padded, 53.9 without.
 template <int N, int XF>
 constexpr bool smooth_pad(int more) {
   return !(XF * Smooth<N, true>::AREA * 8 + more > kSmoothLds3 && XF * Smooth<N, false>::AREA * 8 + more <= kSmoothLds3 &&
