@@ -15,8 +15,8 @@
 // sign: 6.0e-8 against 5.9e-7 at K = 1024.  Where a sum is one product (a diagonal matrix times another) the
 // instruction's own rounding shows: 3.2e-8, at most 1.4e-7, against 2.6e-8 and 6e-8.
 // The matrix rate is what pays for it: 8192 x
-// 1024 x 1024 takes 325 us back to back (515 with v_mfma_f32_32x32x2f32 at 85 % of its peak), 412 GF of bf16
-// products at 1.27 PF; the matrix cores are busy 67 to 68 % of the cycles, at 1.66 to 1.83 GHz by card
+// 1024 x 1024 takes 313 to 328 us back to back (512 with v_mfma_f32_32x32x2f32 at 85 % of its peak), 412 GF of bf16
+// products at 1.26 to 1.32 PF; the matrix cores are busy 67 to 68 % of the cycles, at 1.66 to 1.83 GHz by card
 // (rocprofv3; spread thinner, 52 % busy, it clocked 1.95 GHz and took 390 us against 348), probably the power limit.
 //
 // One kernel computes all four real products: each k-step loads the fragments of the three pieces of
