@@ -135,11 +135,12 @@ struct Split {
 
 // bf16 ends at 2^-133, so operands below 2^-110 lose bits as pieces (operands of 1e-36 lost 5e-5 of the result); the
 // matrix instructions keep denormals.  The loss is at most 2^-133 max(|a|, |b|) for each of the 2 K real products of a
-// sum, or some 2^-149 each where the products are that small, so it shows only in sums that are near that.
-// Each thread keeps the least nonzero and the largest magnitude that it splits.  A
-// workgroup that met an operand below kSmall (without one, products are at least 2^-96), and has a sum (0 counts) below
-// K max(2^-108 |a|, 2^-108 |b|, 2^-118), takes fp32 products; what the others lost is below 2^-24 of the sum.
-constexpr float kSmall = 0x1p-48f;
+// sum, or some 2^-149 each where the products are below 2^-118, so it shows only in sums that are near that.
+// Each thread keeps the least nonzero and the largest magnitude of either operand that it splits.  Where one is below
+// kSmall (without one, products are at least 2^-96) the workgroup compares them: if an operand is below kExact
+// or a product may be below kSumFloor, and a sum (0 counts) is below K max(2^-108 |a|, 2^-108 |b|, 2^-118), it
+// takes fp32 products; what the others lost is below 2^-24 of the sum.
+constexpr float kSmall = 0x1p-48f, kExact = 0x1p-110f;
 constexpr float kSumLimit = 0x1p-108f, kSumFloor = 0x1p-118f;
 struct Range {
   unsigned lo = ~0u;  // least of 2 bits(|x|) - 1 (zero wraps to the largest)
@@ -150,7 +151,27 @@ struct Range {
     lo = min(min(lo, u), v);
     hi = fmaxf(fmaxf(hi, fabsf(x[2 * C])), fabsf(x[2 * C + 1]));
   }
-  __device__ __forceinline__ int small() const { return lo < 2 * __float_as_uint(kSmall) - 1 ? 1 : 0; }
+  __device__ __forceinline__ bool small() const { return lo < 2 * __float_as_uint(kSmall) - 1; }
+  // over the workgroup's waves, through 2 * kThreads / 64 words of LDS
+  __device__ __forceinline__ void reduce(unsigned* lds, int w) {
+#pragma unroll
+    for (int d = 32; d > 0; d /= 2) {
+      lo = min(lo, (unsigned)__shfl_xor((int)lo, d));
+      hi = fmaxf(hi, __shfl_xor(hi, d));
+    }
+    if ((threadIdx.x & 63) == 0) {
+      lds[2 * w] = lo;
+      lds[2 * w + 1] = __float_as_uint(hi);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kThreads / 64; ++i) {
+      lo = min(lo, lds[2 * i]);
+      hi = fmaxf(hi, __uint_as_float(lds[2 * i + 1]));
+    }
+  }
+  // the least nonzero magnitude (infinity where there is none)
+  __device__ __forceinline__ float least() const { return lo == ~0u ? INFINITY : __uint_as_float((lo + 1) / 2); }
 };
 
 __device__ __forceinline__ int outside(float x, float limit) {
@@ -210,8 +231,8 @@ __device__ __forceinline__ void clear(Acc& acc) {
 // The tile's sums with fp32 products (v_mfma_f32_32x32x2f32), k from k_begin to K: the pieces of an
 // infinity are not its sum and those of the smallest numbers may be flushed, so a workgroup whose sums show either
 // (or an overflow) takes this path over, and its results are those of fp32 arithmetic.
-// Two stages in LDS, the next one on its way in registers.  8192 x 1024 x 1024 where every workgroup takes it: 850 us, of which
-// 530 here (with fp32 products alone 512; 880 with one stage in LDS).
+// Two stages in LDS, the next one on its way in registers.  8192 x 1024 x 1024 where every workgroup takes it: 840 us, of which
+// 520 here (with fp32 products alone 512; 868 with one stage in LDS).
 constexpr int GLD = GBM + 2;  // LDS row pitch in floats (pad 2: transposed stores hit distinct banks)
 typedef float F32Stage[2][GBK][GLD];  // [plane][k][row]
 static_assert(2 * kStage >= 4 * (int)sizeof(F32Stage), "staged in the same LDS");
@@ -267,24 +288,23 @@ __device__ __forceinline__ void tile_f32(F32Stage* S, int k_begin, const OpA& A,
   }
 }
 
-// The tile's sums with split products, k from k_begin to K, and the range of the operands that this thread split.
+// The tile's sums with split products, k from k_begin to K, and the ranges of the operands that this thread split.
 template <bool CONJ_B, class OpA, class OpB>
-__device__ __forceinline__ Range tile_split(char* smem, int k_begin, const OpA& A, const OpB& B, int w, Acc& acc_re,
-                                          Acc& acc_im) {
+__device__ __forceinline__ void tile_split(char* smem, int k_begin, const OpA& A, const OpB& B, int w, Acc& acc_re,
+                                           Acc& acc_im, Range& range_a, Range& range_b) {
   const int lane = threadIdx.x & 63, wm = w >> 2, wn = w & 3;
   const int foff = (lane >> 5) * kHalf + (lane & 31) * 16;
   const int a_off = foff + wm * 64 * 16, b_off = kOperand + foff + wn * 32 * 16;
   const int a_dst = A.q.plane * kPlane + A.q.half * kHalf + A.q.row * 16;
   const int b_dst = kOperand + B.q.plane * kPlane + B.q.half * kHalf + B.q.row * 16;
   float xa[8], xb[8];
-  Range range;
   const auto stage = [&](char* S) {
     Split sa, sb;
     unroll<4>([&](auto c) {
       sa.step<c>(xa);
       sb.step<c>(xb);
-      range.pair<c>(xa);
-      range.pair<c>(xb);
+      range_a.pair<c>(xa);
+      range_b.pair<c>(xb);
     });
     sa.store(S + a_dst);
     sb.store(S + b_dst);
@@ -333,8 +353,8 @@ __device__ __forceinline__ Range tile_split(char* smem, int k_begin, const OpA& 
             acc_re[1][r] += re1[r];
           }
         } else {
-          range.pair<s - 8>(xa);
-          range.pair<s - 8>(xb);
+          range_a.pair<s - 8>(xa);
+          range_b.pair<s - 8>(xb);
         }
         __builtin_amdgcn_sched_barrier(0);
       });
@@ -379,7 +399,6 @@ __device__ __forceinline__ Range tile_split(char* smem, int k_begin, const OpA& 
       acc_re[i] += re;
     }
   }
-  return range;
 }
 
 // Operands: A_T = op(A) is a transpose (A stored k x m), B_T = op(B) is one (B stored n x k).  Conjugation:
@@ -422,19 +441,17 @@ __global__ __launch_bounds__(kThreads, SPLIT ? 2 : 4) void cgemm_kernel(
   const Operand<!A_T> A(A_re, A_im, lda, M, K, row0, t, w);
   const Operand<B_T> B(B_re, B_im, ldb, N, K, col0, t, w);
   if constexpr (SPLIT) {
-    const Range range = tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im);
-    // sums below the limit (0 where no operand is small) or not finite need fp32 products
+    Range range_a, range_b;
+    tile_split<CONJ_B>(smem, k_begin, A, B, w, acc_re, acc_im, range_a, range_b);
+    // sums below the limit (0 where nothing is lost) or not finite need fp32 products
     float limit = 0.0f;
-    if (__syncthreads_or(range.small())) {
-      float hi = range.hi;
-#pragma unroll
-      for (int d = 32; d > 0; d /= 2) hi = fmaxf(hi, __shfl_xor(hi, d));
-      float* const wave_hi = reinterpret_cast<float*>(smem);
-      if ((t & 63) == 0) wave_hi[w] = hi;
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < kThreads / 64; ++i) hi = fmaxf(hi, wave_hi[i]);
-      limit = (float)(K - k_begin) * fmaxf(kSumLimit * hi, kSumFloor);
+    if (__syncthreads_or(range_a.small() || range_b.small())) {
+      unsigned* const lds = reinterpret_cast<unsigned*>(smem);
+      range_a.reduce(lds, w);
+      range_b.reduce(lds + 2 * kThreads / 64, w);
+      const float a = range_a.least(), b = range_b.least();
+      if (fminf(a, b) < kExact || a * b < kSumFloor)
+        limit = (float)(K - k_begin) * fmaxf(kSumLimit * fmaxf(range_a.hi, range_b.hi), kSumFloor);
     }
     int odd = 0;
 #pragma unroll
