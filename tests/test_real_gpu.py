@@ -143,3 +143,14 @@ def test_irfft_past_the_completed_length_is_refused_as_before():
     s = ComplexTensor(torch.randn(2, 5).cuda(), torch.randn(2, 5).cuda())
     with pytest.raises(RuntimeError):
         trnfft_amd.irfft(s, n=12)  # the completion has 9 elements at most
+
+
+@pytest.mark.parametrize("on_host", ["real", "imag"])
+@pytest.mark.parametrize("n", [12, 100, 101])
+def test_irfft_of_planes_on_two_devices(n, on_host):
+    # one plane in host memory: copied, never handed to a kernel by its address; the result is on the real plane's device
+    g = torch.Generator().manual_seed(n)
+    re, im = (torch.randn(3, n // 2 + 1, generator=g) for _ in range(2))
+    want = trnfft_amd.irfft(ComplexTensor(re.cuda(), im.cuda()), n=n)
+    got = trnfft_amd.irfft(ComplexTensor(re, im.cuda()) if on_host == "real" else ComplexTensor(re.cuda(), im), n=n)
+    assert got.is_cuda == (on_host == "imag") and torch.equal(got.cuda(), want)

@@ -84,8 +84,8 @@ def irfft(input: ComplexTensor, n: int | None = None) -> torch.Tensor:
         return _ag.c2r(input.real, input.imag, n)
     re, im = input.real, input.imag
     half = re.shape[-1]
-    if (re.is_cuda and re.dtype == torch.float32 == im.dtype and 1 <= half <= n <= 2 * half - 1 and n > 1
-            and not _ag._grad_on(re, im)):
+    if (re.is_cuda and im.device == re.device and re.dtype == torch.float32 == im.dtype
+            and 1 <= half <= n <= 2 * half - 1 and n > 1 and not _ag._grad_on(re, im)):
         # completion and inverse transform, one launch each
         _resolve(None)
         _require_hip("irfft")
