@@ -24,8 +24,8 @@ import torch
 REF = "/root/reference"
 OUT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "bluestein_vectors.npz")
 
-# (n, batch): the reference tests' arbitrary sizes (tests/conftest.py:21-23) plus the two
-# benchmark's Bluestein lengths at small batch.
+# (n, batch): the reference tests' arbitrary sizes (tests/conftest.py:21-23) plus the
+# benchmark's two Bluestein lengths at small batch.
 CASES = [(7, 3), (11, 2), (100, 3), (127, 2), (997, 2), (1000, 4), (4099, 2)]
 
 
